@@ -599,6 +599,10 @@ int bp_slices_per_item(int store, int mode, int variant)
 void launch_backproject(const BpArgs& b, int store, hipStream_t st)
 {
     if (b.S <= 0 || b.n <= 0) return;
+    if (b.chunk == BP_MX || b.chunk == BP_MX_CHECKED) {
+        launch_backproject_mx(b, store, st);
+        return;
+    }
     bp_check_rows(b, store);
     BpKArgs k = bp_kargs(b);
     const int per = bp_slices_per_item(store, b.mode, b.chunk);

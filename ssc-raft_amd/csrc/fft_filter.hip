@@ -227,6 +227,8 @@ struct FilterK {
     const float* wa;
     int N, A, S, npad, L, tlo, W, none;
     int SB; // slices per interleaved group
+    int split; // FP32: entries as three bf16 pieces, [3][W] 8-byte entries per row (the matrix backprojector's)
+    int rg, ra; // row index of (group, angle): g rg + a ra
     float* rows; // k_filter_fft_entry_lds only: non-null -> windows to rows [S][A][W] instead of q
 };
 
@@ -271,12 +273,43 @@ template <> struct Pair2<__half> {
     __device__ static __forceinline__ T make(float a, float b) { return __floats2half2_rn(a, b); }
 };
 
+__device__ __forceinline__ size_t row_index(const FilterK& k, int g, int a)
+{
+    return (size_t)g * k.rg + (size_t)a * k.ra;
+}
+
+// entry w of (group, angle) row `ga`: four slices, as they are or in pieces
+__device__ __forceinline__ void store_entry(const FilterK& k, size_t ga, int w, float4 v)
+{
+    if (k.split) {
+        uint2 h, m, l;
+        split4(v, h, m, l);
+        uint2* d = static_cast<uint2*>(k.q) + ga * 3 * k.W + w;
+        d[0] = h;
+        d[k.W] = m;
+        d[2 * (size_t)k.W] = l;
+    } else {
+        (static_cast<float4*>(k.q) + ga * k.W)[w] = v;
+    }
+}
+
+// two slices of an entry in pieces: words `pr` of the three 8-byte entries
+__device__ __forceinline__ void store_pair_split(const FilterK& k, const PairIdx& ix, int w, float v0, float v1)
+{
+    uint2 h, m, l;
+    split4(make_float4(v0, v1, 0.0f, 0.0f), h, m, l);
+    unsigned* d = static_cast<unsigned*>(k.q) + (row_index(k, ix.g, ix.a) * 3 * k.W + w) * 2 + (ix.s0 - ix.g * 4) / 2;
+    d[0] = h.x;
+    d[2 * (size_t)k.W] = m.x;
+    d[4 * (size_t)k.W] = l.x;
+}
+
 // window store: bins [tlo, tlo + W) of both rows, times the angle weight
 template <typename OT, int THREADS>
 __device__ __forceinline__ void store_pair(const FilterK& k, const PairIdx& ix, const float2* z, float sign1)
 {
     using P2 = typename Pair2<OT>::T;
-    P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(k.q) + (((size_t)ix.g * k.A + ix.a) * k.W) * k.SB +
+    P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(k.q) + (row_index(k, ix.g, ix.a) * k.W) * k.SB +
                                     (ix.s0 - ix.g * k.SB));
     const int stride = k.SB / 2; // in pairs
     const float wv = k.wa[ix.a];
@@ -288,7 +321,8 @@ __device__ __forceinline__ void store_pair(const FilterK& k, const PairIdx& ix, 
             v0 = zv.x * wv;
             v1 = sign1 * zv.y * wv;
         }
-        dst[(size_t)w * stride] = Pair2<OT>::make(v0, v1);
+        if (sizeof(OT) == 4 && k.split) store_pair_split(k, ix, w, v0, v1);
+        else dst[(size_t)w * stride] = Pair2<OT>::make(v0, v1);
     }
 }
 
@@ -364,15 +398,16 @@ __global__ __launch_bounds__(THREADS) void k_filter_fft_entry(FilterK a, FftK p)
             hold[pr][j] = v;
         }
     }
-    uint4* dst = reinterpret_cast<uint4*>(static_cast<OT*>(a.q)) + ((size_t)g * a.A + ang) * a.W;
+    uint4* dst = reinterpret_cast<uint4*>(static_cast<OT*>(a.q)) + row_index(a, g, ang) * a.W;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         const int w = (int)threadIdx.x + j * THREADS;
         if (w >= a.W) continue;
         uint4 e;
         if constexpr (SB == 4) {
-            e = make_uint4(__float_as_uint(hold[0][j].x), __float_as_uint(hold[0][j].y), __float_as_uint(hold[1][j].x),
-                           __float_as_uint(hold[1][j].y));
+            store_entry(a, row_index(a, g, ang), w,
+                        make_float4(hold[0][j].x, hold[0][j].y, hold[1][j].x, hold[1][j].y));
+            continue;
         } else {
             unsigned u[PAIRS];
 #pragma unroll
@@ -405,7 +440,6 @@ __global__ __launch_bounds__(THREADS, WPE) void k_filter_fft_entry_lds(FilterK a
     const int ang = blockIdx.x % a.A, g = blockIdx.x / a.A;
     const float wv = a.wa[ang];
     const float sign1 = a.none ? 1.0f : -1.0f;
-    uint4* dst = reinterpret_cast<uint4*>(static_cast<float*>(a.q)) + ((size_t)g * a.A + ang) * a.W;
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
         const PairIdx ix{g, ang, g * 4 + 2 * pr};
@@ -444,8 +478,7 @@ __global__ __launch_bounds__(THREADS, WPE) void k_filter_fft_entry_lds(FilterK a
                 if (s0 + 3 < a.S) r0[3 * ss] = v.y;
             } else {
                 const float2 h = win[w];
-                dst[w] = make_uint4(__float_as_uint(h.x), __float_as_uint(h.y), __float_as_uint(v.x),
-                                    __float_as_uint(v.y));
+                store_entry(a, row_index(a, g, ang), w, make_float4(h.x, h.y, v.x, v.y));
             }
         }
     }
@@ -465,7 +498,7 @@ __global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
         return;
     }
     using P2 = typename Pair2<OT>::T;
-    P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(a.q) + (((size_t)ix.g * a.A + ix.a) * a.W) * a.SB +
+    P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(a.q) + (row_index(a, ix.g, ix.a) * a.W) * a.SB +
                                     (ix.s0 - ix.g * a.SB));
     const int stride = a.SB / 2;
     const float wv = a.wa[ix.a];
@@ -484,7 +517,8 @@ __global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
                 d = (d == 0) ? a.npad - 1 : d - 1;
             }
         }
-        dst[(size_t)w * stride] = Pair2<OT>::make((float)s0 * wv, (float)s1 * wv);
+        if (sizeof(OT) == 4 && a.split) store_pair_split(a, ix, w, (float)s0 * wv, (float)s1 * wv);
+        else dst[(size_t)w * stride] = Pair2<OT>::make((float)s0 * wv, (float)s1 * wv);
     }
 }
 
@@ -997,6 +1031,9 @@ bool launch_fbp_filter(const FilterArgs& a, const FftPlan& plan, int store, hipS
     k.tomo = a.tomo; k.q = a.q; k.H = a.H; k.tw = a.tw; k.g = a.g; k.wa = a.wa;
     k.N = a.N; k.A = a.A; k.S = a.S; k.npad = a.npad; k.L = a.L; k.tlo = a.tlo; k.W = a.W; k.none = a.none;
     k.SB = (store == RAFT_STORE_F16) ? 8 : 4;
+    k.split = store == RAFT_STORE_F32 ? a.mx : 0;
+    k.rg = a.mx ? 1 : a.A;
+    k.ra = a.mx ? (a.S + k.SB - 1) / k.SB : 1;
     k.rows = store == RAFT_STORE_F32 ? a.rows : nullptr;
     bool direct = false;
     const long long groups = (a.S + k.SB - 1) / k.SB;
@@ -1049,6 +1086,9 @@ void launch_bst(const BstArgs& a, const FftPlan& plan, hipStream_t st, const Fil
         f.N = filt->N; f.A = filt->A; f.S = filt->S; f.npad = n; f.L = filt->L; f.tlo = 0; f.W = n;
         f.none = filt->none;
         f.SB = 4;
+        f.split = 0;
+        f.rg = f.A;
+        f.ra = 1;
         f.rows = nullptr;
         if ((long long)((f.S + f.SB - 1) / f.SB) * f.A * (f.SB / 2) > 0x7fffffffLL)
             fail(RAFT_EUNSUPPORTED, "too many sinogram rows for one BST launch");

@@ -551,30 +551,53 @@ static void fbp_geometry(const FbpCfg& c, const float* angles, BpGeom& g, std::v
     bp_window(g);
 }
 
+// the matrix backprojector's coefficient table: {cA, cB} per angle, the last
+// one repeated for the rounds it reads ahead (BP_MX_TABLE_PAD; its checked form
+// reads none)
+static std::vector<double> paired_coefs(const BpGeom& g, size_t pad = BP_MX_TABLE_PAD)
+{
+    const size_t A = g.cA.size();
+    std::vector<double> v(2 * (A + pad));
+    for (size_t a = 0; a < A + pad; ++a) {
+        v[2 * a] = g.cA[std::min(a, A - 1)];
+        v[2 * a + 1] = g.cB[std::min(a, A - 1)];
+    }
+    return v;
+}
+
 // FBP work of one call on stream st; the caller holds D.mu with the device
 // bound.  sync: wait for the stream before returning (the per-call tables in
 // the arena are then free for the next call).
+// mx: run the matrix form of the backprojector (bp_matrix_form of the whole
+// call; it rounds differently from the gather forms, so all blocks of a call
+// take the same one)
 static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* angles, const FbpCfg& c, int store,
-                    hipStream_t st, bool sync)
+                    hipStream_t st, bool sync, bool mx)
 {
     const int A = c.A, N = c.N;
     BpGeom g;
     std::vector<float> wa;
     fbp_geometry(c, angles, g, wa);
+    if (mx) bp_window_matrix(g);
 
     FilterTables& F = filter_tables(D, c, st);
     TableSet tb(D);
-    const TabRef dcA = tb.add(g.cA), dcB = tb.add(g.cB), dwa = tb.add(wa);
+    const TabRef dcA = tb.add(g.cA), dcB = tb.add(g.cB), dwa = tb.add(wa), dcs = tb.add(paired_coefs(g));
     tb.upload(st);
     if (!sync) tb.keep_alive();
 
     const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
-    const size_t per_group = (size_t)A * g.width * 16; // SB values per bin, 16 bytes
-    // blocks are whole slice groups (except the last)
+    // SB values per bin: 16 bytes, or the matrix form's
+    const size_t per_group = (size_t)A * g.width * (mx ? bp_matrix_entry(store) : 16);
+    // blocks are whole slice groups, packs of the matrix form (except the last)
+    const int BR = mx ? bp_matrix_pack(store) : SB;
     int B = c.blocksize > 0 ? std::min(c.blocksize, c.S) : c.S;
-    B = std::min(c.S, ((B + SB - 1) / SB) * SB);
+    B = std::min(c.S, ((B + BR - 1) / BR) * BR);
     const size_t budget = block_budget();
-    while (B > SB && (size_t)((B + SB - 1) / SB) * per_group > budget) B = (((B + 1) / 2 + SB - 1) / SB) * SB;
+    while (B > SB && (size_t)((B + SB - 1) / SB) * per_group > budget) {
+        const int R = B > BR ? BR : SB;
+        B = (((B + 1) / 2 + R - 1) / R) * R;
+    }
     void* q = D.workspace<0>((size_t)((B + SB - 1) / SB) * per_group);
 
     for (int s0 = 0; s0 < c.S; s0 += B) {
@@ -588,6 +611,7 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
         fa.wa = dwa.as<float>();
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = g.tlo; fa.W = g.width;
         fa.none = (c.filter == 0);
+        fa.mx = mx;
         {
             ProfScope ps(KF_FILTER, st);
             launch_fbp_filter(fa, F.plan, store, st);
@@ -601,14 +625,16 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
         ba.xc = g.xc; ba.c0 = g.c0;
         ba.n = N; ba.A = A; ba.S = nb; ba.tlo = g.tlo; ba.W = g.width; ba.mode = 0;
         ba.q_bytes = (size_t)((B + SB - 1) / SB) * per_group;
+        ba.cs = dcs.as<double>();
         // angle chunk: tuned on this block's rows (the timed launches write
         // the same output as the final one)
-        ba.chunk = tune_pick(bp_tune_key(N, A, g.width, store, 0, (nb + SB - 1) / SB), bp_cands(store), st,
-                             [&](int c) {
-                                 BpArgs t = ba;
-                                 t.chunk = c;
-                                 launch_backproject(t, store, st);
-                             });
+        ba.chunk = mx ? BP_MX
+                      : tune_pick(bp_tune_key(N, A, g.width, store, 0, (nb + SB - 1) / SB), bp_cands(store), st,
+                                  [&](int c) {
+                                      BpArgs t = ba;
+                                      t.chunk = c;
+                                      launch_backproject(t, store, st);
+                                  });
         {
             ProfScope ps(KF_BP, st);
             launch_backproject(ba, store, st);
@@ -629,7 +655,7 @@ static void fbp_device(int dev, float* d_obj, const float* d_tomo, const float* 
     bind_device(dev);
     Device& D = device_state(dev);
     std::lock_guard<std::mutex> lk(D.mu);
-    fbp_run(D, d_obj, d_tomo, angles, c, store, st, true);
+    fbp_run(D, d_obj, d_tomo, angles, c, store, st, true, bp_matrix_form(c.S, c.N, store));
 }
 
 // FBP with every intermediate in the library's fixed device scratch array
@@ -697,6 +723,18 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     int B = c.blocksize > 0 ? std::min(c.blocksize, c.S) : c.S;
     B = std::min(c.S, ((B + SB - 1) / SB) * SB);
     B = std::min(B, groups_fit * SB);
+    // The matrix form where fbp_run takes it, in blocks of whole packs.  Where
+    // the scratch holds fewer than 16 slices its instructions would run mostly
+    // empty (2048 x 2048 FP32: 8 slices fit) and the gather form stays.
+    const int fit = groups_fit * SB;
+    const bool mx = bp_matrix_form(c.S, N, store) && fit >= 16;
+    if (mx) {
+        const int unit = fit >= 2 * bp_matrix_pack(store) ? 2 * bp_matrix_pack(store) : std::min(bp_matrix_pack(store), fit);
+        B = std::min(c.S, std::min(fit, B + unit - 1) / unit * unit);
+        // its coefficient pairs take the place of the two tables
+        const std::vector<double> cs = paired_coefs(g, 0);
+        std::memcpy(host.data() + oA, cs.data(), cs.size() * sizeof(double));
+    }
 
     bind_device(dev);
     Device& D = device_state(dev);
@@ -705,7 +743,10 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     RAFT_HIP(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, st));
     void* q = base + oRows;
     const size_t q_bytes = (size_t)((B + SB - 1) / SB) * per_group;
-    const int chunk = tune_cached(bp_tune_key(N, A, g.width, store, 0, (B + SB - 1) / SB), BP_CHUNK);
+    // the matrix form's checked staging reads the gather forms' rows, so the
+    // scratch holds as many slice groups as for those
+    const int chunk = mx ? BP_MX_CHECKED
+                         : tune_cached(bp_tune_key(N, A, g.width, store, 0, (B + SB - 1) / SB), BP_CHUNK);
 
     for (int s0 = 0; s0 < c.S; s0 += B) {
         const int nb = std::min(B, c.S - s0);
@@ -728,7 +769,8 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
         ba.xc = g.xc; ba.c0 = g.c0;
         ba.n = N; ba.A = A; ba.S = nb; ba.tlo = g.tlo; ba.W = g.width; ba.mode = 0;
         ba.q_bytes = q_bytes;
-        ba.chunk = bp_variant_supported(chunk, store) ? chunk : BP_CHUNK;
+        ba.chunk = mx || bp_variant_supported(chunk, store) ? chunk : BP_CHUNK;
+        ba.cs = mx ? reinterpret_cast<const double*>(base + oA) : nullptr;
         launch_backproject(ba, store, st);
     }
     // the host copy of the tables stays alive until the stream is done
@@ -1935,7 +1977,8 @@ static void fbp_host(int* gpus, int ngpus, float* obj, float* tomo, float* angle
             if (k >= NB) RAFT_HIP(hipStreamWaitEvent(s_comp.s, ev_d2h[b], 0)); // d_out[b] read by chunk k-NB's copy
             FbpCfg ck = c;
             ck.S = nb;
-            fbp_run(D, d_out[b], d_in[b], angles, ck, RAFT_STORE_F32, s_comp.s, false);
+            // gather form: a chunk holds few slices, and the copies bound this path
+            fbp_run(D, d_out[b], d_in[b], angles, ck, RAFT_STORE_F32, s_comp.s, false, false);
             RAFT_HIP(hipEventRecord(ev_comp[b], s_comp.s));
             RAFT_HIP(hipStreamWaitEvent(s_out.s, ev_comp[b], 0));
             // pin_out[b] was copied out (host_out(k - NB)) before this iteration

@@ -77,6 +77,11 @@ constexpr int BP_PAIR = 1024;
 // | BP_SPF: the single form whose sweep loads the next 4 angles' coefficients
 // one trip ahead (fewer registers; same sums bit for bit)
 constexpr int BP_SPF = 2048;
+// the matrix form (backproject_mx.hip), chosen by bp_matrix_form, not timed
+// (BP_MX_CHECKED: from the gather forms' rows, in a fixed scratch)
+constexpr int BP_MX = 4096;
+constexpr int BP_MX_CHECKED = 8192;
+constexpr int BP_MX_TABLE_PAD = 40; // entries its coefficient table repeats past the last angle
 constexpr int BP_GROUP = 16;   // angles per partial sum of the FP32 two-level summation
 constexpr int BP_SLOT = 80;    // LDS entries per staged angle window (>= |(63, 31)| + 5)
 // the pair form's window (two workgroups per CU fit 160 KB of LDS at 32
@@ -89,6 +94,24 @@ constexpr int BP_SLICES_F32 = 4;
 constexpr int BP_SLICES_F16 = 8;
 // projector: consecutive angles per workgroup (one wave each)
 constexpr int PROJ_ANGLES = 8;
+
+// Four FP32 values as three bf16 pieces each, h + m + l exactly (8 significant
+// bits per piece, truncated); piece k of value j sits in 16 bits of word j / 2
+__device__ __forceinline__ void split4(const float4 v, uint2& h, uint2& m, uint2& l)
+{
+    const unsigned u[4] = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+    unsigned r[4], q[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float d = __uint_as_float(u[j]) - __uint_as_float(u[j] & 0xffff0000u);
+        r[j] = __float_as_uint(d);
+        q[j] = __float_as_uint(d - __uint_as_float(r[j] & 0xffff0000u));
+    }
+    // the upper halves of two words, the first in the low half
+    h = make_uint2(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u));
+    m = make_uint2(__builtin_amdgcn_perm(r[1], r[0], 0x07060302u), __builtin_amdgcn_perm(r[3], r[2], 0x07060302u));
+    l = make_uint2(__builtin_amdgcn_perm(q[1], q[0], 0x07060302u), __builtin_amdgcn_perm(q[3], q[2], 0x07060302u));
+}
 
 // global bin window covering every pixel of the tile grid
 void bp_window(BpGeom& g);
@@ -135,6 +158,7 @@ struct FilterArgs {
     const float* wa;    // [A] per-angle weight (dtheta * angular scale)
     int N, A, S, npad, L, tlo, W;
     int none;           // filter 'none': no filtering, no 1/(npad h)
+    int mx = 0;         // rows of the matrix backprojector (bp_matrix_entry)
     float* rows = nullptr; // FP32, W = N: where the kernel form allows, the window is written
                            // straight to rows [S][A][W] (may be tomo itself) instead of q
 };
@@ -177,8 +201,21 @@ struct BpArgs {
     int norm_il = 0;    // mode 1: norm is per slice, interleaved [G][n][n][4] (tEM)
     int chunk = 0;      // variant: angles per LDS round (16, 32 or 48; 0 = 32), | BP_PAIR for the pair form
     size_t q_bytes = 0; // bytes of the buffer behind q when known: launches that would read past it are refused
+    const double* cs = nullptr; // matrix form: {cA, cB} pairs per angle
 };
 void launch_backproject(const BpArgs& a, int store, hipStream_t st);
+// whether an FBP call of S slices of n x n runs the matrix form (chunk =
+// BP_MX); decided once per call, so blocks of a call agree
+bool bp_matrix_form(int S, int n, int store);
+// slices of its smallest pack: blocks of a call are multiples of it
+int bp_matrix_pack(int store);
+// bytes of its rows per (slice group, angle, bin): FP32 rows are staged as
+// [A][G][3][W] 8-byte entries, 4 slices of one bf16 piece (see split4), FP16
+// rows as [A][G][W] 16-byte entries
+size_t bp_matrix_entry(int store);
+// bins its rows hold: every window its tiles stage
+void bp_window_matrix(BpGeom& g);
+void launch_backproject_mx(const BpArgs& b, int store, hipStream_t st);
 // whether variant (see BpArgs::chunk) exists for rows of this store
 bool bp_variant_supported(int variant, int store);
 // slices one workgroup (one queue item) of this variant covers
