@@ -13,15 +13,18 @@
 // reads, zeros outside [0, n), into the slice-interleaved layout
 // [group][angle][bin][SB] (SB = 4 for FP32 rows, 8 for FP16 rows).
 //
-// Padded sizes with a prime factor > 5 or n > 16384 use k_filter_direct:
-// q[m] = sum_j g[(m - j) mod n] u[j] with g = IDFT(H) (built on the host in
-// FP64), the same circular convolution.
+// Padded sizes with a prime factor > 5 or n > 16384 run the same circular
+// convolution q[m] = sum_j g[(m - j) mod n] u[j], g = IDFT(H) (built on the host
+// in FP64), in FP64: by transforms (k_filter_conv) or, for short rows and for
+// rows past its transforms' length, as that sum (k_filter_direct).
 //
 // Reference behaviour restated: paddR2R (padding.cu:140-178), filterFBP /
 // convolution_R2C_C2R_1D / fbp_filtering_R2C2R (filters.cu:33-51,68-87,163-190),
 // Filter::apply (filters.cu:395-438).
 #include "raft_internal.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 namespace raft {
@@ -484,25 +487,28 @@ __global__ __launch_bounds__(THREADS, WPE) void k_filter_fft_entry_lds(FilterK a
     }
 }
 
-// direct circular convolution for sizes the LDS FFT does not cover:
-// q[m] = sum_j g[(m - j) mod n] u[j]
+// bin w of both rows, FP64 sums
 template <typename OT>
-__global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
+__device__ __forceinline__ void store_sum(const FilterK& a, const PairIdx& ix, int w, double s0, double s1)
 {
-    extern __shared__ float2 z[]; // u0 + i u1; the filtered values go straight to the staged rows
-    const PairIdx ix = pair_index(a);
-    load_pair<256>(a, ix, z);
-    __syncthreads();
-    if (a.none) {
-        store_pair<OT, 256>(a, ix, z, 1.0f);
-        return;
-    }
-    using P2 = typename Pair2<OT>::T;
-    P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(a.q) + (row_index(a, ix.g, ix.a) * a.W) * a.SB +
-                                    (ix.s0 - ix.g * a.SB));
-    const int stride = a.SB / 2;
     const float wv = a.wa[ix.a];
-    for (int w = threadIdx.x; w < a.W; w += 256) {
+    const float v0 = (float)s0 * wv, v1 = (float)s1 * wv;
+    if (sizeof(OT) == 4 && a.split) {
+        store_pair_split(a, ix, w, v0, v1);
+    } else {
+        using P2 = typename Pair2<OT>::T;
+        P2* dst = reinterpret_cast<P2*>(static_cast<OT*>(a.q) + (row_index(a, ix.g, ix.a) * a.W) * a.SB +
+                                        (ix.s0 - ix.g * a.SB));
+        dst[(size_t)w * (a.SB / 2)] = Pair2<OT>::make(v0, v1);
+    }
+}
+
+// direct circular convolution for sizes the LDS FFT does not cover:
+// q[m] = sum_j g[(m - j) mod n] u[j], bins [w0, w1) of the pair in z
+template <typename OT, int THREADS>
+__device__ __forceinline__ void direct_window(const FilterK& a, const PairIdx& ix, const float2* z, int w0, int w1)
+{
+    for (int w = w0 + (int)threadIdx.x; w < w1; w += THREADS) {
         const int T = a.tlo + w;
         // FP64 kernel and sums: the kernel sums to ~0 (no DC), so n FP32
         // products would lose ~sqrt(n) ulps of a cancelling sum
@@ -517,9 +523,289 @@ __global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
                 d = (d == 0) ? a.npad - 1 : d - 1;
             }
         }
-        if (sizeof(OT) == 4 && a.split) store_pair_split(a, ix, w, (float)s0 * wv, (float)s1 * wv);
-        else dst[(size_t)w * stride] = Pair2<OT>::make((float)s0 * wv, (float)s1 * wv);
+        store_sum<OT>(a, ix, w, s0, s1);
     }
+}
+
+template <typename OT>
+__global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
+{
+    extern __shared__ float2 z[]; // u0 + i u1; the filtered values go straight to the staged rows
+    const PairIdx ix = pair_index(a);
+    load_pair<256>(a, ix, z);
+    __syncthreads();
+    if (a.none) {
+        store_pair<OT, 256>(a, ix, z, 1.0f);
+        return;
+    }
+    direct_window<OT, 256>(a, ix, z, 0, a.W);
+}
+
+// ---- the same convolution by FP64 transforms (k_filter_conv) --------------
+//
+// q[T] = sum_{i < N} g[(T - L - i) mod n] r[i] + r[0] e0[T] + r[N - 1] e1[T]: the
+// padding's constant runs are two tables of partial sums of g, the interior is a
+// linear convolution of N samples.  A workgroup computes `chunk` outputs of two
+// rows (one complex signal: the kernel is real) with transforms of
+// len >= N + chunk - 1 in LDS: decimation in frequency forward, the product with
+// the kernel's spectrum in the order that leaves, decimation in time back, so
+// nothing is reordered.  Passes of radix 8 in registers, the first reads the
+// rows, the last writes the bins; one complex of padding per 8 keeps the passes'
+// strides off each other's banks.  FP64 throughout, like the direct form: an
+// FP32 transform's rounding (1e-6) would be ten times this path's error.
+//
+// What bounds it: twiddles and spectrum from L2 (16 bytes each; three twiddles a
+// butterfly, the others their products) and LDS passes.  21 slices of 901 x 1301
+// padded to 2602 (len 4096): 0.36 ms, the direct sum 22.7 (n x window products a
+// row); 8 of 300 x 2047 padded to 6141 (len 8192): 0.13 against 9.7.
+constexpr int CV_THREADS = 512;
+constexpr int CV_MAX_LEN = 8192; // 147 KB of LDS
+constexpr int CV_MAX_CHUNKS = 16;
+// padded rows from here on: n = 98 takes 10.2 us direct and 13.6 by transforms
+// (320 row pairs), n = 202 43.7 and 22.8 (1440 pairs)
+constexpr int CV_MIN_N = 128;
+typedef double d2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ int cpix(int e) { return e + (e >> 3); }
+size_t conv_lds(int len) { return sizeof(double) * 2 * ((size_t)len + (size_t)(len >> 3) + 1); }
+
+struct ConvK {
+    const d2* spec;     // [chunks][len], permuted as the forward passes leave it, 1 / len folded in
+    const d2* tw;       // [len] exp(-2 pi i k / len)
+    const double* edge; // [2][n]: e0, e1
+    int len, chunk, first, count; // outputs per chunk; first chunk and chunks of this launch
+    int passes, radix[8];
+    unsigned rows; // (group, angle) pairs
+};
+
+__device__ __forceinline__ d2 zmul(d2 a, d2 b)
+{
+    return d2{fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
+}
+__device__ __forceinline__ d2 zconj(d2 a) { return d2{a.x, -a.y}; }
+// a * -i (forward), a * i (inverse)
+template <bool INV> __device__ __forceinline__ d2 zrot(d2 a) { return INV ? d2{-a.y, a.x} : d2{a.y, -a.x}; }
+
+template <bool INV> __device__ __forceinline__ void zdft4(d2& a, d2& b, d2& c, d2& d)
+{
+    const d2 s = a + c, t = a - c, u = b + d, v = zrot<INV>(b - d);
+    a = s + u; b = t + v; c = s - u; d = t - v;
+}
+// DFT of v[0..R) in place, W = exp(-+ 2 pi i / R)
+template <int R, bool INV> __device__ __forceinline__ void zdft(d2 (&v)[R])
+{
+    static_assert(R == 3 || R == 4 || R == 5 || R == 8, "radix");
+    if constexpr (R == 3) {
+        const double h = 0.86602540378443864676; // sin 60 degrees
+        const d2 s = v[1] + v[2], m = v[0] - 0.5 * s, r = zrot<INV>(h * (v[1] - v[2]));
+        v[0] = v[0] + s; v[1] = m + r; v[2] = m - r;
+    } else if constexpr (R == 4) {
+        zdft4<INV>(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 5) {
+        const double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410; // cos 72, cos 144 degrees
+        const double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;  // their sines
+        const d2 p1 = v[1] + v[4], p2 = v[2] + v[3], q1 = v[1] - v[4], q2 = v[2] - v[3];
+        const d2 m1 = v[0] + c1 * p1 + c2 * p2, m2 = v[0] + c2 * p1 + c1 * p2;
+        const d2 r1 = zrot<INV>(s1 * q1 + s2 * q2), r2 = zrot<INV>(s2 * q1 - s1 * q2);
+        v[0] = v[0] + p1 + p2;
+        v[1] = m1 + r1; v[4] = m1 - r1; v[2] = m2 + r2; v[3] = m2 - r2;
+    } else {
+        const double h = 0.70710678118654752440; // sqrt(1/2)
+        zdft4<INV>(v[0], v[2], v[4], v[6]);
+        zdft4<INV>(v[1], v[3], v[5], v[7]);
+        // odd part times W_8^k, k = 0..3 (in v[1], v[3], v[5], v[7])
+        const d2 o1 = h * (v[3] + zrot<INV>(v[3])), o2 = zrot<INV>(v[5]), o3 = h * (zrot<INV>(v[7]) - v[7]);
+        const d2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
+        v[0] = e0 + o0; v[4] = e0 - o0;
+        v[1] = e1 + o1; v[5] = e1 - o1;
+        v[2] = e2 + o2; v[6] = e2 - o2;
+        v[3] = e3 + o3; v[7] = e3 - o3;
+    }
+}
+// v[q] *= W_len^(x q) (conjugate for the inverse)
+template <int R, bool INV> __device__ __forceinline__ void ztwiddle(d2 (&v)[R], const d2* tw, int x)
+{
+    d2 w[R];
+    w[1] = tw[x];
+    w[2] = tw[2 * x];
+    if constexpr (R > 4) w[4] = tw[4 * x];
+    if constexpr (R > 3) w[3] = zmul(w[1], w[2]);
+    if constexpr (R > 5) {
+        w[5] = zmul(w[1], w[4]);
+        w[6] = zmul(w[2], w[4]);
+        w[7] = zmul(w[3], w[4]);
+    }
+#pragma unroll
+    for (int q = 1; q < R; ++q) v[q] = zmul(v[q], INV ? zconj(w[q]) : w[q]);
+}
+
+// the first forward pass, from the rows; returns whether a sample read is not finite
+template <int R>
+__device__ __forceinline__ bool conv_first(const FilterK& a, const PairIdx& ix, const ConvK& c, d2* z)
+{
+    const bool h0 = ix.s0 < a.S, h1 = ix.s0 + 1 < a.S;
+    const float* r0 = a.tomo + ((size_t)ix.s0 * a.A + ix.a) * a.N;
+    const float* r1 = r0 + (size_t)a.A * a.N;
+    const int M = c.len / R;
+    bool bad = false;
+    for (int j = threadIdx.x; j < M; j += CV_THREADS) {
+        d2 v[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const int i = j + t * M;
+            const float x0 = h0 && i < a.N ? r0[i] : 0.0f, x1 = h1 && i < a.N ? r1[i] : 0.0f;
+            bad |= !((x0 - x0) + (x1 - x1) == 0.0f);
+            v[t] = d2{(double)x0, (double)x1};
+        }
+        zdft<R, false>(v);
+        ztwiddle<R, false>(v, c.tw, j);
+#pragma unroll
+        for (int t = 0; t < R; ++t) z[cpix(j + t * M)] = v[t];
+    }
+    return bad;
+}
+// a pass over blocks of B elements
+template <int R, bool INV> __device__ __forceinline__ void conv_pass(const ConvK& c, int B, d2* z)
+{
+    const int M = B / R, lm = 31 - __clz(M), step = c.len / B; // M is a power of two
+    for (int b = threadIdx.x; b < c.len / R; b += CV_THREADS) {
+        const int j = b & (M - 1), base = (b >> lm) * B + j;
+        d2 v[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) v[t] = z[cpix(base + t * M)];
+        if (INV) ztwiddle<R, true>(v, c.tw, step * j);
+        zdft<R, INV>(v);
+        if (!INV) ztwiddle<R, false>(v, c.tw, step * j);
+#pragma unroll
+        for (int t = 0; t < R; ++t) z[cpix(base + t * M)] = v[t];
+    }
+}
+// the last inverse pass, to the bins
+template <typename OT, int R>
+__device__ __forceinline__ void conv_last(const FilterK& a, const PairIdx& ix, const ConvK& c, int T0, const d2* z)
+{
+    const float* r0 = a.tomo + ((size_t)ix.s0 * a.A + ix.a) * a.N;
+    const float* r1 = r0 + (size_t)a.A * a.N;
+    const bool h0 = ix.s0 < a.S, h1 = ix.s0 + 1 < a.S;
+    const double l0 = h0 ? r0[0] : 0.0f, l1 = h1 ? r1[0] : 0.0f;
+    const double u0 = h0 ? r0[a.N - 1] : 0.0f, u1 = h1 ? r1[a.N - 1] : 0.0f;
+    const int M = c.len / R;
+    const int lo = max(T0, a.tlo), hi = min(min(T0 + c.chunk, a.npad), a.tlo + a.W); // this chunk's bins
+    for (int j = threadIdx.x; j < M; j += CV_THREADS) {
+        d2 v[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) v[t] = z[cpix(j + t * M)];
+        ztwiddle<R, true>(v, c.tw, j);
+        zdft<R, true>(v);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const int T = T0 + j + t * M;
+            if (T < lo || T >= hi) continue;
+            const double e0 = c.edge[T], e1 = c.edge[a.npad + T];
+            store_sum<OT>(a, ix, T - a.tlo, fma(u0, e1, fma(l0, e0, v[t].x)), fma(u1, e1, fma(l1, e0, v[t].y)));
+        }
+    }
+}
+
+template <typename OT> __global__ __launch_bounds__(CV_THREADS, 4) void k_filter_conv(FilterK a, ConvK c)
+{
+    extern __shared__ __align__(16) char conv_smem[];
+    d2* z = reinterpret_cast<d2*>(conv_smem);
+    // the pairs and chunks of a row on one XCD (workgroups go to the 8 XCDs round
+    // robin): their interleaved stores share cache lines
+    const unsigned per = (unsigned)(a.SB / 2) * c.count;
+    const unsigned ga = (blockIdx.x >> 3) / per * 8u + (blockIdx.x & 7u);
+    if (ga >= c.rows) return;
+    const unsigned sub = (blockIdx.x >> 3) % per;
+    PairIdx ix;
+    ix.a = (int)(ga % (unsigned)a.A);
+    ix.g = (int)(ga / (unsigned)a.A);
+    ix.s0 = ix.g * a.SB + 2 * (int)(sub / c.count);
+    const int ch = c.first + (int)(sub % c.count);
+    const int T0 = ch * c.chunk;
+    // bins outside [0, n) are zero: the launch's first and last chunk clear them
+    if (ch == c.first)
+        for (int w = threadIdx.x; w < min(-a.tlo, a.W); w += CV_THREADS) store_sum<OT>(a, ix, w, 0.0, 0.0);
+    if (ch == c.first + c.count - 1)
+        for (int w = max(a.npad - a.tlo, 0) + (int)threadIdx.x; w < a.W; w += CV_THREADS)
+            store_sum<OT>(a, ix, w, 0.0, 0.0);
+    if (ix.s0 >= a.S) { // padding slices of the last group
+        for (int T = max(T0, a.tlo) + (int)threadIdx.x; T < min(min(T0 + c.chunk, a.npad), a.tlo + a.W); T += CV_THREADS)
+            store_sum<OT>(a, ix, T - a.tlo, 0.0, 0.0);
+        return;
+    }
+
+    bool bad;
+    switch (c.radix[0]) {
+    case 3: bad = conv_first<3>(a, ix, c, z); break;
+    case 4: bad = conv_first<4>(a, ix, c, z); break;
+    case 5: bad = conv_first<5>(a, ix, c, z); break;
+    default: bad = conv_first<8>(a, ix, c, z); break;
+    }
+    if (__syncthreads_or(bad)) {
+        // a row that is not finite must not reach the other of the pair
+        load_pair<CV_THREADS>(a, ix, reinterpret_cast<float2*>(z));
+        __syncthreads();
+        direct_window<OT, CV_THREADS>(a, ix, reinterpret_cast<const float2*>(z), max(T0 - a.tlo, 0),
+                                      min(min(T0 + c.chunk, a.npad) - a.tlo, a.W));
+        return;
+    }
+    int B = c.len / c.radix[0];
+    int p = 1;
+    for (; p < c.passes - 1; ++p) {
+        if (c.radix[p] == 4) conv_pass<4, false>(c, B, z);
+        else conv_pass<8, false>(c, B, z);
+        B /= c.radix[p];
+        __syncthreads();
+    }
+    // the last forward pass (radix 8, blocks of 8: no twiddles), the product and
+    // the first inverse pass in registers
+    const d2* spec = c.spec + (size_t)ch * c.len;
+    for (int b = threadIdx.x; b < c.len / 8; b += CV_THREADS) {
+        d2 v[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) v[t] = z[cpix(8 * b) + t];
+        zdft<8, false>(v);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) v[t] = zmul(v[t], spec[8 * b + t]);
+        zdft<8, true>(v);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) z[cpix(8 * b) + t] = v[t];
+    }
+    __syncthreads();
+    for (p = c.passes - 2; p > 0; --p) {
+        B *= c.radix[p];
+        if (c.radix[p] == 4) conv_pass<4, true>(c, B, z);
+        else conv_pass<8, true>(c, B, z);
+        __syncthreads();
+    }
+    switch (c.radix[0]) {
+    case 3: conv_last<OT, 3>(a, ix, c, T0, z); break;
+    case 4: conv_last<OT, 4>(a, ix, c, T0, z); break;
+    case 5: conv_last<OT, 5>(a, ix, c, T0, z); break;
+    default: conv_last<OT, 8>(a, ix, c, T0, z); break;
+    }
+}
+
+template <typename OT> void launch_conv(const FilterK& k, const FilterArgs& a, hipStream_t st)
+{
+    const ConvPlan& p = a.conv;
+    ConvK c;
+    c.spec = static_cast<const d2*>(a.conv_spec);
+    c.tw = static_cast<const d2*>(a.conv_tw);
+    c.edge = a.conv_edge;
+    c.len = p.len; c.chunk = p.chunk; c.passes = p.passes;
+    std::copy(p.radix, p.radix + 8, c.radix);
+    // chunks that hold bins of the window (one at least, for the zeros outside [0, n))
+    const int lo = std::min(std::max(k.tlo, 0), k.npad - 1), hi = std::min(std::max(k.tlo + k.W, 1), k.npad);
+    c.first = lo / p.chunk;
+    c.count = std::max((hi - 1) / p.chunk - c.first + 1, 1);
+    c.rows = (unsigned)((long long)((k.S + k.SB - 1) / k.SB) * k.A);
+    const long long blocks = ((long long)c.rows + 7) / 8 * 8 * (k.SB / 2) * c.count;
+    if (blocks > 0x7fffffffLL) fail(RAFT_EUNSUPPORTED, "too many sinogram rows for one filter launch");
+    const size_t lds = std::max(conv_lds(p.len), sizeof(float2) * lds_elems(k.npad));
+    RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_filter_conv<OT>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_filter_conv<OT>), dim3((unsigned)blocks), dim3(CV_THREADS), lds, st, k, c);
 }
 
 template <typename OT, int THREADS, int E>
@@ -1024,6 +1310,101 @@ FftPlan fft_plan(int n)
     return p;
 }
 
+ConvPlan conv_plan(int n, int N)
+{
+    ConvPlan best;
+    if (n < CV_MIN_N) return best;
+    long long cost = 0;
+    for (int m : {1, 3, 5})
+        for (int len = m * 64, k = 6; len <= CV_MAX_LEN; len *= 2, ++k) {
+            const int chunk = std::min(len - N + 1, n);
+            if (chunk < 1) continue;
+            const int chunks = (n + chunk - 1) / chunk;
+            if (best.len && (long long)chunks * len >= cost) continue;
+            cost = (long long)chunks * len;
+            best = ConvPlan();
+            best.len = len; best.chunk = chunk; best.chunks = chunks;
+            if (m > 1) best.radix[best.passes++] = m;
+            const int fours = k % 3 == 0 ? 0 : (k % 3 == 2 ? 1 : 2);
+            for (int i = 0; i < fours; ++i) best.radix[best.passes++] = 4;
+            for (int i = 0; i < (k - 2 * fours) / 3; ++i) best.radix[best.passes++] = 8;
+        }
+    if (best.chunks > CV_MAX_CHUNKS) best = ConvPlan();
+    return best;
+}
+
+void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::vector<double>& spec,
+                 std::vector<double>& tw, std::vector<double>& edge)
+{
+    const int len = p.len;
+    std::vector<double> w(2 * (size_t)len);
+    for (int k = 0; k < len; ++k) {
+        const double ang = -2.0 * M_PI * (double)k / (double)len;
+        w[2 * k] = std::cos(ang);
+        w[2 * k + 1] = std::sin(ang);
+    }
+    // frequency held at each position after the forward passes: position
+    // q (block / radix) + r holds radix f(r) + q
+    std::vector<int> freq(1, 0);
+    for (int i = p.passes - 1; i >= 0; --i) {
+        std::vector<int> up;
+        for (int q = 0; q < p.radix[i]; ++q)
+            for (int f : freq) up.push_back(p.radix[i] * f + q);
+        freq.swap(up);
+    }
+    spec.assign(2 * (size_t)len * p.chunks, 0.0);
+    std::vector<double> x(2 * (size_t)len), y(2 * (size_t)len);
+    for (int c = 0; c < p.chunks; ++c) {
+        std::fill(x.begin(), x.end(), 0.0);
+        const long long T0 = (long long)c * p.chunk;
+        for (int t = -(N - 1); t < p.chunk; ++t)
+            x[2 * (size_t)((t + len) % len)] = g[(((T0 + t - L) % n) + n) % n] / (double)len;
+        // forward transform, radix-2 steps down to the odd factor (decimation in time)
+        int m = len;
+        while (m % 2 == 0) m /= 2;
+        const int q = len / m; // q interleaved transforms of length m
+        for (int r = 0; r < q; ++r)
+            for (int k = 0; k < m; ++k) {
+                double re = 0.0, im = 0.0;
+                for (int i = 0; i < m; ++i) {
+                    const size_t e = 2 * ((size_t)r + (size_t)q * i), f = 2 * (size_t)((long long)i * k % m * q);
+                    re += x[e] * w[f] - x[e + 1] * w[f + 1];
+                    im += x[e] * w[f + 1] + x[e + 1] * w[f];
+                }
+                y[2 * ((size_t)r * m + k)] = re;
+                y[2 * ((size_t)r * m + k) + 1] = im;
+            }
+        // y: [r][k], transforms of x[r + q i]; pairs r, r + h combine to length 2 s
+        for (int h = q / 2, s = m; h >= 1; h /= 2, s *= 2) {
+            for (int r = 0; r < h; ++r)
+                for (int k = 0; k < s; ++k) {
+                    const double* e = &y[2 * ((size_t)r * s + k)];
+                    const double* o = &y[2 * ((size_t)(r + h) * s + k)];
+                    const double* f = &w[2 * (size_t)k * h];
+                    const double re = o[0] * f[0] - o[1] * f[1], im = o[0] * f[1] + o[1] * f[0];
+                    double* d0 = &x[2 * ((size_t)r * 2 * s + k)];
+                    double* d1 = &x[2 * ((size_t)r * 2 * s + k + s)];
+                    d0[0] = e[0] + re; d0[1] = e[1] + im;
+                    d1[0] = e[0] - re; d1[1] = e[1] - im;
+                }
+            x.swap(y);
+        }
+        for (int e = 0; e < len; ++e) {
+            spec[2 * ((size_t)c * len + e)] = y[2 * (size_t)freq[e]];
+            spec[2 * ((size_t)c * len + e) + 1] = y[2 * (size_t)freq[e] + 1];
+        }
+    }
+    tw = w;
+    edge.assign(2 * (size_t)n, 0.0);
+    for (int T = 0; T < n; ++T) {
+        double e0 = 0.0, e1 = 0.0;
+        for (int j = 0; j < L; ++j) e0 += g[(T - j + n) % n];
+        for (int j = L + N; j < n; ++j) e1 += g[(T - j + n) % n];
+        edge[T] = e0;
+        edge[(size_t)n + T] = e1;
+    }
+}
+
 bool launch_fbp_filter(const FilterArgs& a, const FftPlan& plan, int store, hipStream_t st)
 {
     if (a.S <= 0 || a.A <= 0) return a.rows != nullptr && store == RAFT_STORE_F32;
@@ -1048,7 +1429,10 @@ bool launch_fbp_filter(const FilterArgs& a, const FftPlan& plan, int store, hipS
         else direct = launch_fft<float>(k, p, threads, (int)blocks, lds_fft, st);
     } else {
         if (lds > 160 * 1024) fail(RAFT_EUNSUPPORTED, "padded row too long for the direct filter path");
-        if (store == RAFT_STORE_F16) {
+        if (a.conv.len > 0) {
+            if (store == RAFT_STORE_F16) launch_conv<__half>(k, a, st);
+            else launch_conv<float>(k, a, st);
+        } else if (store == RAFT_STORE_F16) {
             RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_filter_direct<__half>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             hipLaunchKernelGGL((k_filter_direct<__half>), dim3((int)blocks), dim3(256), lds, st, k);

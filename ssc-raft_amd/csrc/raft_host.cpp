@@ -296,7 +296,19 @@ static double filter_apply(int type, double w, double reg, double pag)
 // ---------------------------------------------------------------------------
 struct FilterTables {
     DevBuf H, tw, g; // float2[n], float2[n], double[n]
+    DevBuf spec, ctw, edge; // see conv_tables
     FftPlan plan;
+    ConvPlan conv;
+    void set(FilterArgs& a) const
+    {
+        a.H = static_cast<const float2*>(H.p);
+        a.tw = static_cast<const float2*>(tw.p);
+        a.g = static_cast<const double*>(g.p);
+        a.conv = conv;
+        a.conv_spec = spec.p;
+        a.conv_tw = ctw.p;
+        a.conv_edge = static_cast<const double*>(edge.p);
+    }
 };
 
 // page-locked host buffer (hipHostMalloc), grow-only
@@ -447,8 +459,9 @@ template <typename T> static void upload(DevBuf& b, const std::vector<T>& v, hip
 // the real convolution kernel g
 struct FilterHost {
     std::vector<float2> H, tw;
-    std::vector<double> g;
+    std::vector<double> g, spec, ctw, edge;
     FftPlan plan;
+    ConvPlan conv;
 };
 
 static void filter_host_tables(const FbpCfg& c, FilterHost& F)
@@ -495,15 +508,17 @@ static void filter_host_tables(const FbpCfg& c, FilterHost& F)
             }
             F.g[d] = acc;
         }
+        F.conv = conv_plan(n, c.N);
+        if (F.conv.len) conv_tables(F.conv, F.g.data(), n, c.N, c.L, F.spec, F.ctw, F.edge);
     }
 }
 
-// the key of a filter table set: (n, filter, reg, paganin, offset, pixel)
+// the key of a filter table set: (n, N, L, filter, reg, paganin, offset, pixel)
 static std::string filter_key(const FbpCfg& c)
 {
     char key[256];
-    snprintf(key, sizeof key, "%d/%d/%.17g/%.17g/%.17g/%.17g", c.npad, c.filter, c.reg, c.paganin, c.offset,
-             c.pixel);
+    snprintf(key, sizeof key, "%d/%d/%d/%d/%.17g/%.17g/%.17g/%.17g", c.npad, c.N, c.L, c.filter, c.reg, c.paganin,
+             c.offset, c.pixel);
     return key;
 }
 
@@ -520,6 +535,12 @@ static FilterTables& filter_tables(Device& D, const FbpCfg& c, hipStream_t st)
     upload(F->H, h.H, st);
     upload(F->tw, h.tw, st);
     if (!h.g.empty()) upload(F->g, h.g, st);
+    F->conv = h.conv;
+    if (h.conv.len) {
+        upload(F->spec, h.spec, st);
+        upload(F->ctw, h.ctw, st);
+        upload(F->edge, h.edge, st);
+    }
     RAFT_HIP(hipStreamSynchronize(st));
     auto& ref = *F;
     D.filters[key] = std::move(F);
@@ -605,9 +626,7 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
         FilterArgs fa;
         fa.tomo = d_tomo + (size_t)s0 * A * N;
         fa.q = q;
-        fa.H = F.H.as<float2>();
-        fa.tw = F.tw.as<float2>();
-        fa.g = F.g.as<double>();
+        F.set(fa);
         fa.wa = dwa.as<float>();
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = g.tlo; fa.W = g.width;
         fa.none = (c.filter == 0);
@@ -707,14 +726,21 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     const size_t oH = put(F->H.data(), F->H.size() * sizeof(float2));
     const size_t oTw = put(F->tw.data(), F->tw.size() * sizeof(float2));
     const size_t oG = put(F->g.data(), F->g.size() * sizeof(double));
+    // the convolution form's tables, where a slice group of rows still fits
+    // behind them (else the direct sum of the same FP64 terms)
+    const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
+    const size_t per_group = (size_t)A * g.width * 16;
+    const size_t cap = (size_t)RAFT_NOALLOC_SCRATCH_BYTES;
+    const size_t conv_bytes = (F->spec.size() + F->ctw.size() + F->edge.size()) * sizeof(double) + 3 * 256;
+    const bool conv = F->conv.len > 0 && host.size() + conv_bytes + (size_t)A * 20 + 4 * 256 + per_group <= cap;
+    const size_t oSpec = conv ? put(F->spec.data(), F->spec.size() * sizeof(double)) : 0;
+    const size_t oCtw = conv ? put(F->ctw.data(), F->ctw.size() * sizeof(double)) : 0;
+    const size_t oEdge = conv ? put(F->edge.data(), F->edge.size() * sizeof(double)) : 0;
     const size_t oA = put(g.cA.data(), (size_t)A * sizeof(double));
     const size_t oB = put(g.cB.data(), (size_t)A * sizeof(double));
     const size_t oW = put(wa.data(), (size_t)A * sizeof(float));
     const size_t oRows = (host.size() + 255) & ~(size_t)255;
 
-    const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
-    const size_t per_group = (size_t)A * g.width * 16;
-    const size_t cap = (size_t)RAFT_NOALLOC_SCRATCH_BYTES;
     if (oRows > cap || cap - oRows < per_group)
         fail(RAFT_EUNSUPPORTED, "raft_fbp_device_noalloc: tables (" + std::to_string(oRows) +
                                     " bytes) and one slice group of filtered rows (" + std::to_string(per_group) +
@@ -756,6 +782,12 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
         fa.H = reinterpret_cast<const float2*>(base + oH);
         fa.tw = reinterpret_cast<const float2*>(base + oTw);
         fa.g = F->g.empty() ? nullptr : reinterpret_cast<const double*>(base + oG);
+        if (conv) {
+            fa.conv = F->conv;
+            fa.conv_spec = base + oSpec;
+            fa.conv_tw = base + oCtw;
+            fa.conv_edge = reinterpret_cast<const double*>(base + oEdge);
+        }
         fa.wa = reinterpret_cast<const float*>(base + oW);
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = g.tlo; fa.W = g.width;
         fa.none = (c.filter == 0);
@@ -890,9 +922,7 @@ static void lowpass_device(int dev, float* d_tomo, const float* paramf, const in
         FilterArgs fa;
         fa.tomo = d_tomo + (size_t)s0 * A * N;
         fa.q = q;
-        fa.H = F.H.as<float2>();
-        fa.tw = F.tw.as<float2>();
-        fa.g = F.g.as<double>();
+        F.set(fa);
         fa.wa = dwa.as<float>();
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = c.L; fa.W = N;
         fa.none = 0;
@@ -1488,9 +1518,7 @@ static void batch_device(int dev, int nscans, const int* nrays, const int* nangl
             FilterArgs fa;
             fa.tomo = b->tomo.as<float>();
             fa.q = b->frows.p;
-            fa.H = b->F->H.as<float2>();
-            fa.tw = b->F->tw.as<float2>();
-            fa.g = b->F->g.as<double>();
+            b->F->set(fa);
             fa.wa = b->fwa.as<float>();
             fa.N = N; fa.A = A; fa.S = S; fa.npad = b->cf.npad; fa.L = b->cf.L; fa.tlo = b->gf.tlo; fa.W = b->gf.width;
             fa.none = (b->cf.filter == 0);

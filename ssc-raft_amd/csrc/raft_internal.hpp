@@ -149,12 +149,28 @@ struct FftPlan {
 };
 FftPlan fft_plan(int n);
 
+// transforms of the convolution form (sizes without an FftPlan); len 0: the direct sum
+struct ConvPlan {
+    int len = 0, chunk = 0, chunks = 0; // transform length, outputs per transform, transforms covering [0, n)
+    int passes = 0;
+    int radix[8] = {0};
+};
+ConvPlan conv_plan(int n, int N);
+// its tables from the circular kernel g[n]: spectra [chunks][len] and twiddles
+// [len] (complex), edge sums [2][n]
+void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::vector<double>& spec,
+                 std::vector<double>& tw, std::vector<double>& edge);
+
 struct FilterArgs {
     const float* tomo;  // [S][A][N]
     void* q;            // [G][A][W][SB] float (SB = 4) or __half (SB = 8)
     const float2* H;    // [npad] Hermitian filter incl. 1/(npad*pixel)
     const float2* tw;   // two-level twiddles: lo[128] = W^k, hi[npad/128 + 1] = W^(128k), W = exp(-2 pi i/npad)
     const double* g;    // direct-convolution kernel (real, [npad], FP64) or null
+    ConvPlan conv;      // len > 0: with the three tables below (see conv_tables)
+    const void* conv_spec = nullptr;
+    const void* conv_tw = nullptr;
+    const double* conv_edge = nullptr;
     const float* wa;    // [A] per-angle weight (dtheta * angular scale)
     int N, A, S, npad, L, tlo, W;
     int none;           // filter 'none': no filtering, no 1/(npad h)
