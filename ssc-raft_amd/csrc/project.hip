@@ -7,7 +7,7 @@
 // interleaved transpose instead, so the fast-varying direction across rays is
 // always the contiguous one.
 //
-// Two forms share the sampling and the epilogue:
+// Three forms share the sampling and the epilogue:
 //
 // Staged form (k_project_lds, dense angle sets).  One workgroup = 8 waves =
 // 8 consecutive angles, one ray chunk, one slice group.  The waves walk the
@@ -37,10 +37,11 @@
 // staged after the barrier, as in the plain form.  Both forms stage the same
 // values, so they agree bit for bit.
 // The host admits a launch to this form only when every chunk's union box
-// fits PL_CAP entries at every patch position (proj_plan); sparse angle sets
-// use the direct form.
+// fits PL_CAP entries at every patch position (proj_plan).
 //
-// Direct form (k_project): one workgroup per (block of PROJ_ANGLES
+// Tile form (k_project_tile, k_project_sum; sparse angle sets): below.
+//
+// Direct form (k_project; images below 32 x 32, stretched pixels): one workgroup per (block of PROJ_ANGLES
 // consecutive angles, slice group), one wave per angle.  The waves walk the
 // same blocks of R consecutive rays in lockstep (a barrier per block), so the
 // 8 nearby angles read nearly the same image region at the same time and the
@@ -341,6 +342,207 @@ __global__ __launch_bounds__(64 * PROJ_ANGLES, 4) void k_project(ProjK a)
         __syncthreads(); // keep the waves (angles) of the workgroup on the same ray block
     }
     if (EM == 1 && a.kl_part && have) kl_flush(a, g, ang, lane, klsum, exc, kp, min(Kp, 4));
+}
+
+// ---- tile form ----
+//
+// Sparse angle sets share no image region between neighbouring angles, so the
+// direct form reads every sample from L2.  Here a workgroup stages one tile of
+// PT_T x PT_T pixels of a slice group in LDS and sums, for a range of angles, the
+// samples of every ray that fall into it; k_project_sum adds a ray's partial sums
+// over the tiles it crosses, in a fixed order, and forms the output.  A wave
+// takes one angle: 16 neighbouring rays x 4 samples at a time.
+//
+// Rays of a tile: the sampling grid is a rotation (ry rx = 1), so ray index is
+// affine in the pixel; the rays within `half` of the tile's centre hold all its
+// samples (margins of 1.5 pixels, as truncation takes (-1, 0) to pixel 0), and
+// both kernels number them from pt_first.  Samples are taken from a generous
+// range of k and tested exactly, in integers, against the tile.
+//
+// A wave's lane takes ray lane / 4 of 16 neighbouring ones and every fourth
+// sample.  Row pitch 4 mod 16: the 16 entries of an LDS pass, 4 rays x 4 samples,
+// fall on distinct bank groups (X + 4 Y) when the patch lies along the axes.
+//
+// What bounds it: vector operations, twelve for a sample's place (five in FP64)
+// and four for its sums.  Two slice groups share the places where there are two
+// (their rows side by side; 16 waves, 136 KB, one workgroup per CU; one group: 8 waves, two workgroups).
+// Tiles of 64 keep the partial sums at 1.3 / 64 of the samples.
+//
+// Projection, direct form -> this one: 6 slices of 700 x 500, 90 angles 0.76 ->
+// 0.071 ms; 64 of 512 x 512, 128 angles 0.66 -> 0.37; 8 of 2048 x 2048, 180 angles
+// 8.6 -> 1.10.  Where the staged form is admitted it is faster (512 angles of 16
+// slices of 512 x 512: 0.31 against 0.35; 2048 of 32 of 2048 x 2048: 31 against 45).
+constexpr int PT_T = 64;
+
+struct TileK {
+    float4* part;       // [groups of the launch][tile][angle of the launch][rs]
+    int tx, ty;         // tiles
+    int rs;             // partial sums per (tile, angle)
+    int a0, na, per;    // first angle, angles of the launch, angles per workgroup
+    int g0, ng;         // first slice group, groups of the launch
+};
+
+struct TileRays {
+    double cs, bxk, byi, half;
+    int count;
+    __device__ __forceinline__ TileRays(const ProjK& a, int ang)
+    {
+        cs = a.cosv[ang];
+        const double sn = a.sinv[ang];
+        bxk = -sn * a.ry;
+        byi = sn * a.rx;
+        half = (fabs(cs) + fabs(bxk)) * (0.5 * PT_T + 1.5);
+        count = (int)(2.0 * half) + 3;
+    }
+    __device__ __forceinline__ double centre(const ProjK& a, int tx, int ty) const
+    {
+        const double dx = (double)(tx * PT_T + PT_T / 2) - a.ucx, dy = (double)(ty * PT_T + PT_T / 2) - a.ucy;
+        return fma(cs, dx, fma(-bxk, dy, a.ci));
+    }
+    __device__ __forceinline__ int first(const ProjK& a, int tx, int ty) const
+    {
+        return (int)floor(centre(a, tx, ty) - half);
+    }
+};
+
+// sum over a lane's group of four
+__device__ __forceinline__ float quad_sum(float v)
+{
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)); // quad_perm 1 0 3 2
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)); // quad_perm 2 3 0 1
+    return v;
+}
+
+// NG: slice groups per workgroup
+template <int NG> __global__ __launch_bounds__(512 * NG, 4) void k_project_tile(ProjK a, TileK t)
+{
+    constexpr int THREADS = 512 * NG, WAVES = THREADS / 64;
+    constexpr int ROW = NG == 1 ? 68 : 66, PITCH = NG * ROW, ZERO = PT_T * PITCH; // entries; ZERO: zeros
+    __shared__ float4 tile[ZERO + (NG - 1) * ROW + 1];
+    const int tx = blockIdx.x % t.tx, ty = blockIdx.x / t.tx, g0 = blockIdx.z * NG;
+    const int X0 = tx * PT_T, Y0 = ty * PT_T;
+    const size_t plane = (size_t)a.Nx * a.Ny;
+#pragma unroll
+    for (int u = 0; u < PT_T * PT_T / 512; ++u) {
+        const int e = (int)threadIdx.x + u * THREADS;
+        const int x = e % PT_T, y = e / PT_T % PT_T, g = e / (PT_T * PT_T);
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (X0 + x < a.Nx && Y0 + y < a.Ny && g0 + g < t.ng)
+            v = a.img[(size_t)(t.g0 + g0 + g) * plane + (size_t)(Y0 + y) * a.Nx + X0 + x];
+        tile[y * PITCH + g * ROW + x] = v;
+    }
+    if (threadIdx.x < NG) tile[ZERO + threadIdx.x * ROW] = make_float4(0.f, 0.f, 0.f, 0.f);
+    __syncthreads();
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane >> 2, kp = lane & 3;
+    const int ax0 = blockIdx.y * t.per, ax1 = min(ax0 + t.per, t.na);
+    const size_t gstep = (size_t)t.tx * t.ty * t.na * t.rs; // partial sums of a group
+    for (int ax = ax0 + wave; ax < ax1; ax += WAVES) {
+        const TileRays q(a, t.a0 + ax);
+        const int first = q.first(a, tx, ty);
+        // slopes too small to divide by leave the range of k to the other coordinate
+        const double ib = fabs(q.bxk) > 1.0e-6 ? 1.0 / q.bxk : 0.0, ic = fabs(q.cs) > 1.0e-6 ? 1.0 / q.cs : 0.0;
+        float4* dst = t.part + g0 * gstep + ((size_t)blockIdx.x * t.na + ax) * t.rs;
+        for (int rb = 0; rb < q.count; rb += 16) {
+            const int i = first + rb + r;
+            const bool have = rb + r < q.count && (unsigned)i < (unsigned)a.nrays;
+            const double ir = (double)i - a.ci;
+            const double uxi = fma(ir, q.cs, a.ucx), uyi = fma(ir, q.byi, a.ucy);
+            double klo = 0.0, khi = (double)a.nk;
+            if (ib != 0.0) {
+                const double u = ((double)X0 - 1.5 - uxi) * ib, v = ((double)(X0 + PT_T) + 1.5 - uxi) * ib;
+                klo = fmax(klo, a.ck + fmin(u, v));
+                khi = fmin(khi, a.ck + fmax(u, v));
+            }
+            if (ic != 0.0) {
+                const double u = ((double)Y0 - 1.5 - uyi) * ic, v = ((double)(Y0 + PT_T) + 1.5 - uyi) * ic;
+                klo = fmax(klo, a.ck + fmin(u, v));
+                khi = fmin(khi, a.ck + fmax(u, v));
+            }
+            int cnt = 0; // this lane's samples: k0 + kp, k0 + kp + 4, ...
+            double kr = 0.0;
+            if (have && khi >= klo) {
+                const int k0 = (int)fmax(floor(klo), 0.0) + kp, k1 = (int)fmin(ceil(khi) + 1.0, (double)a.nk);
+                cnt = (k1 - k0 + 3) >> 2;
+                kr = (double)k0 - a.ck;
+            }
+            float4 acc[NG];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) acc[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+            double krs[2] = {kr, kr + 4.0};
+            for (int m = 0; m < cnt; m += 2) {
+                int e[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const unsigned X = (unsigned)((int)fma(krs[u], q.bxk, uxi) - X0);
+                    const unsigned Y = (unsigned)((int)fma(krs[u], q.cs, uyi) - Y0);
+                    const bool in = max(X, Y) < (unsigned)PT_T && m + u < cnt;
+                    e[u] = in ? (int)(__umul24(Y, PITCH) + X) : ZERO;
+                    krs[u] += 8.0; // exact
+                }
+#pragma unroll
+                for (int g = 0; g < NG; ++g) acc[g] = add4(acc[g], add4(tile[e[0] + g * ROW], tile[e[1] + g * ROW]));
+            }
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const float4 v = make_float4(quad_sum(acc[g].x), quad_sum(acc[g].y), quad_sum(acc[g].z), quad_sum(acc[g].w));
+                if (kp == 0 && have && g0 + g < t.ng) dst[g * gstep + rb + r] = v;
+            }
+        }
+    }
+}
+
+// A ray's partial sums over its tiles, along the axis its tiles lie closest to.
+// With KL terms one workgroup takes all rays of an angle, so that the angle's KL
+// partial is summed in a fixed order.
+template <int EM> __global__ __launch_bounds__(256) void k_project_sum(ProjK a, TileK t)
+{
+    const int ax = blockIdx.y, g = blockIdx.z;
+    const TileRays q(a, t.a0 + ax);
+    const bool wide = fabs(q.cs) >= fabs(q.bxk); // a step of tx moves the ray index most
+    const double d = wide ? PT_T * q.cs : -PT_T * q.bxk;
+    const double id = 1.0 / d, reach = fabs((q.half + 2.0) * id);
+    const int no = wide ? t.ty : t.tx, ni = wide ? t.tx : t.ty;
+    const float4* part = t.part + ((size_t)g * t.tx * t.ty * t.na + ax) * t.rs;
+    double kl[4] = {0.0, 0.0, 0.0, 0.0};
+    unsigned ex[4] = {0, 0, 0, 0};
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < a.nrays; i += gridDim.x * 256) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int o = 0; o < no; ++o) {
+            const double at = ((double)i - (wide ? q.centre(a, 0, o) : q.centre(a, o, 0))) * id;
+            const int lo = (int)fmax(ceil(at - reach), 0.0), hi = (int)fmin(floor(at + reach), (double)(ni - 1));
+            for (int n = lo; n <= hi; ++n) {
+                const int tx = wide ? n : o, ty = wide ? o : n;
+                const int s = i - q.first(a, tx, ty);
+                if ((unsigned)s < (unsigned)q.count) acc = add4(acc, part[(size_t)(ty * t.tx + tx) * t.na * t.rs + s]);
+            }
+        }
+        ray_out<EM>(a, t.g0 + g, t.a0 + ax, i, acc, kl, ex);
+    }
+    if (EM == 1 && a.kl_part) {
+        __shared__ double sd[4][4];
+        __shared__ unsigned se[4][4];
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            for (int off = 32; off > 0; off >>= 1) {
+                kl[s] += __shfl_xor(kl[s], off);
+                ex[s] += __shfl_xor(ex[s], off);
+            }
+            if (lane == 0) {
+                sd[wave][s] = kl[s];
+                se[wave][s] = ex[s];
+            }
+        }
+        __syncthreads();
+        const int s = threadIdx.x, sl = (t.g0 + g) * 4 + s;
+        if (s < 4 && sl < a.S) {
+            a.kl_part[(size_t)sl * a.kl_stride + t.a0 + ax] = ((sd[0][s] + sd[1][s]) + sd[2][s]) + sd[3][s];
+            a.ex_part[(size_t)sl * a.kl_stride + t.a0 + ax] =
+                (unsigned long long)se[0][s] + se[1][s] + se[2][s] + se[3][s];
+        }
+    }
 }
 
 // ---- staged form ----
@@ -861,6 +1063,75 @@ void launch_project_queue(const void* d_descs, const ProjQueue& q, int em_mode, 
                              dim3(64 * PROJ_ANGLES), args, 0, st));
 }
 
+static size_t tile_bytes(const RayGeom& g, int rs)
+{
+    const size_t tx = (size_t)(g.Nx + PT_T - 1) / PT_T, ty = (size_t)(g.Ny + PT_T - 1) / PT_T;
+    return tx * ty * (size_t)rs * sizeof(float4); // per (slice group, angle)
+}
+
+int proj_tile_plan(const RayGeom& g, const double* c, const double* s)
+{
+    const char* env = std::getenv("RAFT_PROJ_LDS");
+    if (env && env[0] == '0') return 0;
+    // below, the second launch costs more than the tiles save (16 x 16, 5 angles:
+    // 8.8 us direct, 9.5; 32 x 32, 16 angles: 14.8 and 11.9)
+    if ((long long)g.Nx * g.Ny < 1024) return 0;
+    double w = 0.0;
+    for (int a = 0; a < g.nangles; ++a) w = std::max(w, std::fabs(c[a]) + std::fabs(s[a] * g.ry));
+    const double half = w * (0.5 * PT_T + 1.5);
+    if (!(half < 128.0)) return 0; // stretched pixels: few samples a ray and tile
+    return ((int)(2.0 * half) + 3 + 3) / 4 * 4;
+}
+
+size_t proj_tile_workspace(const RayGeom& g, int rs, int S, size_t cap)
+{
+    if (rs <= 0) return 0;
+    const size_t one = tile_bytes(g, rs), all = one * g.nangles * ((size_t)(S + 3) / 4);
+    const size_t least = one * std::min(g.nangles, 8);
+    return least > cap ? 0 : std::min(all, cap);
+}
+
+static void launch_tiles(const ProjArgs& p, const ProjK& k, int em_mode, int G, hipStream_t st)
+{
+    TileK t;
+    t.part = reinterpret_cast<float4*>(p.tile_part);
+    t.tx = (k.Nx + PT_T - 1) / PT_T;
+    t.ty = (k.Ny + PT_T - 1) / PT_T;
+    t.rs = p.tile_rs;
+    // (group, angle) sums the workspace holds: whole groups, or two groups' angles in turns
+    const size_t fit = p.tile_bytes / tile_bytes(p.g, p.tile_rs);
+    if (fit < 1) fail(RAFT_EINVAL, "internal: the tile projector has no workspace");
+    int gc = (int)std::min<size_t>(fit / (size_t)k.nangles, (size_t)G), ac = k.nangles;
+    if (gc < std::min(G, 2)) {
+        gc = (int)std::min<size_t>(fit, (size_t)std::min(G, 2));
+        ac = (int)std::min<size_t>(fit / gc, (size_t)k.nangles);
+    } else if (gc < G) {
+        gc &= ~1; // pairs of groups
+    }
+    const int tiles = t.tx * t.ty;
+    for (t.g0 = 0; t.g0 < G; t.g0 += gc)
+        for (t.a0 = 0; t.a0 < k.nangles; t.a0 += ac) {
+            t.ng = std::min(gc, G - t.g0);
+            t.na = std::min(ac, k.nangles - t.a0);
+            // two groups a workgroup where that still fills the chip twice (128 x 128,
+            // 60 angles, 8 slices: 20 us with one, 28 with two; 700 x 500, 90 angles, 6
+            // slices: 89 and 73); angles per workgroup: 64 (staging a tile costs as much
+            // as 2), fewer where the chip would not fill four times
+            const int pairs = (t.ng + 1) / 2;
+            const int NG = t.ng > 1 && (long long)tiles * pairs * ((t.na + 15) / 16) >= 512 ? 2 : 1;
+            const int gz = (t.ng + NG - 1) / NG;
+            t.per = 64;
+            while (t.per > 8 * NG && (long long)tiles * gz * ((t.na + t.per - 1) / t.per) < 2048 / NG) t.per /= 2;
+            const dim3 tg(tiles, (t.na + t.per - 1) / t.per, gz);
+            if (NG == 2) hipLaunchKernelGGL((k_project_tile<2>), tg, dim3(1024), 0, st, k, t);
+            else hipLaunchKernelGGL((k_project_tile<1>), tg, dim3(512), 0, st, k, t);
+            const dim3 grid(k.kl_part ? 1 : (k.nrays + 255) / 256, t.na, t.ng);
+            if (em_mode == 2) hipLaunchKernelGGL((k_project_sum<2>), grid, dim3(256), 0, st, k, t);
+            else if (em_mode) hipLaunchKernelGGL((k_project_sum<1>), grid, dim3(256), 0, st, k, t);
+            else hipLaunchKernelGGL((k_project_sum<0>), grid, dim3(256), 0, st, k, t);
+        }
+}
+
 void launch_project(const ProjArgs& p, int em_mode, hipStream_t st)
 {
     if (p.S <= 0 || p.g.nrays <= 0 || p.g.nangles <= 0) return;
@@ -884,6 +1155,8 @@ void launch_project(const ProjArgs& p, int em_mode, hipStream_t st)
             else if (em_mode) hipLaunchKernelGGL((k_project_lds<1, 0>), grid, block, 0, st, k);
             else hipLaunchKernelGGL((k_project_lds<0, 0>), grid, block, 0, st, k);
         }
+    } else if (p.tile_rs > 0) {
+        launch_tiles(p, k, em_mode, G, st);
     } else {
         const dim3 grid(nab, G);
         if (em_mode == 2) hipLaunchKernelGGL((k_project<2>), grid, block, 0, st, k);

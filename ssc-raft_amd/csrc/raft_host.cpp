@@ -342,7 +342,7 @@ struct PinnedBuf {
 };
 
 struct Device {
-    static constexpr int kSlots = 14;
+    static constexpr int kSlots = 15;
     std::mutex mu;
     std::map<std::string, std::unique_ptr<FilterTables>> filters;
     DevBuf ws[kSlots];
@@ -939,6 +939,21 @@ static void lowpass_device(int dev, float* d_tomo, const float* paramf, const in
     RAFT_HIP(hipStreamSynchronize(st));
 }
 
+// tile form of the projector where the angles are too sparse to stage: its
+// workspace is at most PROJ_TILE_CAP and an eighth of the block budget
+constexpr size_t PROJ_TILE_CAP = (size_t)128 << 20;
+static void proj_tiles(Device& D, ProjArgs& p, const std::vector<double>& c, const std::vector<double>& s, int prc, int S,
+                       size_t budget)
+{
+    if (prc > 0) return;
+    const int rs = proj_tile_plan(p.g, c.data(), s.data());
+    const size_t bytes = proj_tile_workspace(p.g, rs, S, std::min(PROJ_TILE_CAP, budget / 8));
+    if (!bytes) return;
+    p.tile_rs = rs;
+    p.tile_part = D.workspace<14>(bytes);
+    p.tile_bytes = bytes;
+}
+
 static void radon_device(int dev, float* d_proj, const float* d_obj, const float* angles, int Nx, int Ny, int nrays,
                          int nangles, int nslices, float ax, float ay, hipStream_t st)
 {
@@ -972,13 +987,14 @@ static void radon_device(int dev, float* d_proj, const float* d_obj, const float
     for (int s0 = 0; s0 < nslices; s0 += B) {
         const int nb = std::min(B, nslices - s0);
         const float* src = d_obj + (size_t)s0 * img;
-        launch_to_interleaved(src, il, nb, Ny, Nx, false, st);
-        launch_to_interleaved(src, ilT, nb, Ny, Nx, true, st);
         ProjArgs p;
         p.img = il; p.imgT = ilT; p.out = d_proj + (size_t)s0 * nangles * nrays;
         p.y = nullptr; p.wa = nullptr; p.kl_part = nullptr; p.ex_part = nullptr;
         p.cosv = dc.as<double>(); p.sinv = ds.as<double>();
         p.g = g; p.S = nb; p.tlo = 0; p.W = nrays; p.lds_rc = prc;
+        proj_tiles(D, p, cv, sv, prc, nb, budget);
+        launch_to_interleaved(src, il, nb, Ny, Nx, false, st);
+        if (!p.tile_rs) launch_to_interleaved(src, ilT, nb, Ny, Nx, true, st); // tiles read one orientation
         if (prc > 0)
             p.lds_rc = tune_pick(proj_tune_key(g, 0, (nb + 3) / 4), proj_rc_cands(g, prc), st, [&](int c) {
                 ProjArgs t = p;
@@ -1108,6 +1124,11 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
     // ratio rows: margins stay zero, the projector writes [0, R) (none for the KL alone)
     if (!kl_only) RAFT_HIP(hipMemsetAsync(rows, 0, (size_t)Gb * A * g.width * 16, st));
 
+    ProjArgs tiles; // the tile form's fields
+    tiles.g = rg;
+    proj_tiles(D, tiles, cv, sv, prc, B, budget);
+    const bool need_T = !tiles.tile_rs; // tiles read one orientation
+
     // one iteration: projector + ratio (+ KL partials), KL reduction, backprojection + update
     int* counter = reinterpret_cast<int*>(static_cast<char*>(D.workspace<6>(256)));
     auto iteration = [&](int it, int nb, const float* y, double* klo, unsigned long long* exo, bool graph,
@@ -1118,6 +1139,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
         p.ex_part = with_kl ? expart : nullptr;
         p.cosv = dc.as<double>(); p.sinv = ds.as<double>();
         p.g = rg; p.S = nb; p.tlo = g.tlo; p.W = g.width; p.lds_rc = prc;
+        p.tile_rs = tiles.tile_rs; p.tile_part = tiles.tile_part; p.tile_bytes = tiles.tile_bytes;
         {
             ProfScope ps(KF_PROJ, s);
             launch_project(p, 1, s);
@@ -1125,7 +1147,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
         if (with_kl) launch_kl_reduce(part, expart, kslots, nb, klo, exo, Kkl, it, graph ? counter : nullptr, s);
         if (kl_only) return;
         BpArgs b;
-        b.q = rows; b.out = xil; b.x = xil; b.norm = ones; b.xt = xT;
+        b.q = rows; b.out = xil; b.x = xil; b.norm = ones; b.xt = need_T ? xT : nullptr;
         b.cA = dcA.as<double>(); b.cB = dcB.as<double>(); b.xc = g.xc; b.c0 = g.c0;
         b.n = n; b.A = A; b.S = nb; b.tlo = g.tlo; b.W = g.width; b.mode = 1; b.chunk = bp_chunk;
         b.q_bytes = (size_t)Gb * A * g.width * 16;
@@ -1184,7 +1206,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
         double* klo = Kkl > 0 ? dkl + (size_t)s0 * Kkl : nullptr;
         unsigned long long* exo = Kkl > 0 ? dex + (size_t)s0 * Kkl : nullptr;
         launch_to_interleaved(x, xil, nb, n, n, false, st);
-        launch_to_interleaved(x, xT, nb, n, n, true, st);
+        if (need_T) launch_to_interleaved(x, xT, nb, n, n, true, st);
         if (s0 == 0) tune(nb, y);
         for (int it = 0; it < it0; ++it) iteration(it, nb, y, klo, exo, false, st, true);
         if (use_graph) {
@@ -1306,6 +1328,10 @@ static void tem_device(int dev, float* d_obj, const float* d_count, const float*
     float* tmp = static_cast<float*>(D.workspace<5>((size_t)B * img * 4));
     const int prc = proj_plan(rg, cv.data(), sv.data(), B, true);
 
+    ProjArgs tiles;
+    tiles.g = rg;
+    proj_tiles(D, tiles, cv, sv, prc, B, budget);
+
     for (int s0 = 0; s0 < S; s0 += B) {
         const int nb = std::min(B, S - s0);
         float* x = d_obj + (size_t)s0 * img;
@@ -1321,19 +1347,20 @@ static void tem_device(int dev, float* d_obj, const float* d_count, const float*
         // the rows' margins (bins outside [0, R)) are zero from here on: the
         // projector rewrites only [0, R)
         launch_to_interleaved(x, xil, nb, n, n, false, st);
-        launch_to_interleaved(x, xT, nb, n, n, true, st);
+        if (!tiles.tile_rs) launch_to_interleaved(x, xT, nb, n, n, true, st);
         for (int it = 0; it < K; ++it) {
             ProjArgs p;
             p.img = xil; p.imgT = xT; p.out = rows; p.y = d_flat + (size_t)s0 * R; p.wa = dwa.as<float>();
             p.kl_part = nullptr; p.ex_part = nullptr;
             p.cosv = dc.as<double>(); p.sinv = ds.as<double>();
             p.g = rg; p.S = nb; p.tlo = g.tlo; p.W = g.width; p.lds_rc = prc;
+            p.tile_rs = tiles.tile_rs; p.tile_part = tiles.tile_part; p.tile_bytes = tiles.tile_bytes;
             {
                 ProfScope ps(KF_PROJ, st);
                 launch_project(p, 2, st);
             }
             BpArgs b;
-            b.q = rows; b.out = xil; b.x = xil; b.norm = normil; b.norm_il = 1; b.xt = xT;
+            b.q = rows; b.out = xil; b.x = xil; b.norm = normil; b.norm_il = 1; b.xt = tiles.tile_rs ? nullptr : xT;
             b.cA = dcA.as<double>(); b.cB = dcB.as<double>(); b.xc = g.xc; b.c0 = g.c0;
             b.n = n; b.A = A; b.S = nb; b.tlo = g.tlo; b.W = g.width; b.mode = 1;
             b.q_bytes = (size_t)Gb * A * g.width * 16;
@@ -1368,7 +1395,8 @@ struct BatchBucket {
     BpGeom ge;
     RayGeom rg;
     int prc = 0; // staged projector plan (ray chunks), 0 = direct form
-    DevBuf dc, ds, ecA, ecB, ewa, erows, xil, xT, ones, y, x;
+    int tile_rs = 0; // tile projector plan (sparse angles)
+    DevBuf dc, ds, ecA, ecB, ewa, erows, xil, xT, ones, y, x, ptile;
     hipStream_t s = nullptr;
     hipEvent_t done = nullptr;
 };
@@ -1464,6 +1492,13 @@ static void batch_device(int dev, int nscans, const int* nrays, const int* nangl
             upload(b->ewa, wa, st);
             b->rg = ray_geom_em(N, A, N);
             b->prc = proj_plan(b->rg, cv.data(), sv.data(), S, true);
+            if (b->prc == 0) {
+                b->tile_rs = proj_tile_plan(b->rg, cv.data(), sv.data());
+                const size_t bytes = proj_tile_workspace(b->rg, b->tile_rs, S,
+                                                         std::min(PROJ_TILE_CAP, block_budget() / (8 * buckets.size())));
+                if (bytes) b->ptile.alloc(bytes);
+                else b->tile_rs = 0;
+            }
             const int G = (S + 3) / 4;
             b->erows.alloc((size_t)G * A * g.width * 16);
             b->xil.alloc((size_t)G * img * 16);
@@ -1496,6 +1531,7 @@ static void batch_device(int dev, int nscans, const int* nrays, const int* nangl
         p.y = b->y.as<float>(); p.wa = b->ewa.as<float>(); p.kl_part = nullptr; p.ex_part = nullptr;
         p.cosv = b->dc.as<double>(); p.sinv = b->ds.as<double>();
         p.g = b->rg; p.S = (int)b->scans.size(); p.tlo = b->ge.tlo; p.W = b->ge.width; p.lds_rc = b->prc;
+        p.tile_rs = b->tile_rs; p.tile_part = b->ptile.p; p.tile_bytes = b->ptile.bytes;
         return p;
     };
     auto em_bp_args = [&](BatchBucket* b) {

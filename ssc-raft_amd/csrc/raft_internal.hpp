@@ -277,7 +277,10 @@ struct ProjArgs {
     RayGeom g;
     int S;
     int tlo, W;         // eEM ratio-row layout
-    int lds_rc = 0;     // > 0: staged form with this many ray chunks (from proj_plan); 0: direct form
+    int lds_rc = 0;     // > 0: staged form with this many ray chunks (from proj_plan); 0: tile or direct form
+    int tile_rs = 0;    // > 0 (from proj_tile_plan): tile form, with its workspace
+    void* tile_part = nullptr;
+    size_t tile_bytes = 0;
 };
 // em_mode 0 = Radon, 1 = eEM ratio (+ KL), 2 = tEM flat * exp(-v).
 // KL partials: kl_part[s * proj_kl_slots(a) + slot], reduced by launch_kl_reduce.
@@ -286,6 +289,11 @@ void launch_project(const ProjArgs& a, int em_mode, hipStream_t st);
 // chunks, or 0 when a chunk of 8 angles cannot be staged (sparse angles) or
 // RAFT_PROJ_LDS=0.  have_T: the transposed image will be passed as imgT.
 int proj_plan(const RayGeom& g, const double* c, const double* s, int S, bool have_T);
+// Tile-form plan for geometries without a staged one: partial sums per (tile,
+// angle), 0 for the direct form (stretched pixels, RAFT_PROJ_LDS=0).
+int proj_tile_plan(const RayGeom& g, const double* c, const double* s);
+// its workspace for S slices, at most cap (launches then run in turns); 0: cap is too small
+size_t proj_tile_workspace(const RayGeom& g, int rs, int S, size_t cap);
 // persistent work-queue form of the staged projector (see BpQueue); segment b
 // has nab[b] angle chunks x RC ray chunks x slice groups items
 struct ProjQueue {
