@@ -50,6 +50,8 @@ struct BpKArgs {
     int n, A, tlo, W, S;
     int tiles_x;
     int norm_il;
+    float* part = nullptr; // MODE 2: sums of BP_GROUP angles each [groups of angles][S][n][n]
+    int per = 0;           // MODE 2: angles of a workgroup (whole groups)
 };
 
 // accumulate one 16-byte staged entry into SB running sums
@@ -142,8 +144,9 @@ __device__ __forceinline__ void bp_tile(const BpKArgs& a, int tile, int gp, BpSm
 #pragma unroll
             for (int s = 0; s < SB; ++s) tot[q][p][s] = 0.0f;
 
-    for (int a0 = 0; a0 < a.A; a0 += CHUNK) {
-        const int nA = __builtin_amdgcn_readfirstlane(min(CHUNK, a.A - a0)); // uniform: scalar loop counter
+    const int alo = MODE == 2 ? (int)blockIdx.z * a.per : 0, ahi = MODE == 2 ? min(a.A, alo + a.per) : a.A;
+    for (int a0 = alo; a0 < ahi; a0 += CHUNK) {
+        const int nA = __builtin_amdgcn_readfirstlane(min(CHUNK, ahi - a0)); // uniform: scalar loop counter
         __syncthreads();
         // ---- per-angle bin windows of this tile (one thread per angle) ----
         if (tid < nA) {
@@ -266,7 +269,18 @@ __device__ __forceinline__ void bp_tile(const BpKArgs& a, int tile, int gp, BpSm
                     }
                 }
             }
-            if constexpr (TWO_LEVEL) {
+            if constexpr (MODE == 2) {
+                float* dst = a.part + (size_t)((a0 + ag) / BP_GROUP) * a.S * a.n * a.n;
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+#pragma unroll
+                        for (int s = 0; s < SB; ++s) {
+                            const int sl = g * SB1 + s, i = i0 + tx + 16 * p, j = j0 + ty + 16 * q;
+                            if (sl < a.S && i < a.n && j < a.n) dst[((size_t)sl * a.n + j) * a.n + i] = part[q][p][s];
+                        }
+            } else if constexpr (TWO_LEVEL) {
 #pragma unroll
                 for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -277,6 +291,7 @@ __device__ __forceinline__ void bp_tile(const BpKArgs& a, int tile, int gp, BpSm
         }
     }
 
+    if (MODE == 2) return;
     // ---- epilogue ----
     const size_t nn = (size_t)a.n * a.n;
 #pragma unroll
@@ -330,6 +345,28 @@ __global__ __launch_bounds__(256, PAIR) void k_backproject(BpKArgs a)
 {
     __shared__ BpSmem<CHUNK, PAIR> sm;
     bp_tile<QT, MODE, CHUNK, PAIR, SPF>(a, blockIdx.x, blockIdx.y, sm);
+}
+
+// Sums of the angle groups in order: the total of a split launch
+__global__ __launch_bounds__(256) void k_bp_groups(const float* part, float* out, int groups, size_t count)
+{
+    const size_t e = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (e + 4 <= count) {
+        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int g = 0; g < groups; ++g) {
+            float v[4]; // count need not be a multiple of 4: 4-byte aligned loads
+            __builtin_memcpy(v, part + (size_t)g * count + e, 16);
+            t = make_float4(t.x + v[0], t.y + v[1], t.z + v[2], t.w + v[3]);
+        }
+        __builtin_memcpy(out + e, &t, 16);
+    } else {
+        for (size_t f = e; f < count; ++f) {
+            float t = 0.0f;
+            for (int g = 0; g < groups; ++g) t += part[(size_t)g * count + f];
+            out[f] = t;
+        }
+    }
 }
 
 // Persistent work-queue form: a resident grid takes items from a device
@@ -533,6 +570,39 @@ static BpKArgs bp_kargs(const BpArgs& b)
     return k;
 }
 
+// Split form of the FBP sums, for calls whose tiles do not fill the chip: the
+// angles of a tile are dealt to several workgroups, which leave the sums of
+// their groups of BP_GROUP angles in a workspace, and k_bp_groups adds those in
+// the order of the whole sum, so the result is the same bit for bit.
+// What bounds the whole form there is the serial walk over the angles by one
+// workgroup on half of the CUs.  1 slice of 512 x 512, 512 angles: 159 us whole,
+// 59 split (about 2048 workgroups; 62 at 768); 4 slices 159 and 80 (134 MB of
+// partial sums); 256 x 256, 256 angles 84 and 16; 64 x 64, 64 angles 24 and 12.
+// Above 256 tiles every CU has work (1024 x 1024: 512 tiles).
+constexpr size_t BP_SPLIT_CAP = (size_t)192 << 20;
+
+size_t bp_split_workspace(int S, int n, int A, int store)
+{
+    const long long wgs = (long long)bp_tiles(n) * ((S + 3) / 4);
+    const size_t bytes = (size_t)((A + BP_GROUP - 1) / BP_GROUP) * S * n * n * sizeof(float);
+    if (store != RAFT_STORE_F32 || wgs > 256 || A < 4 * BP_GROUP || bytes > BP_SPLIT_CAP) return 0;
+    return bytes;
+}
+
+static void launch_backproject_split(const BpArgs& b, BpKArgs k, hipStream_t st)
+{
+    const int groups = (b.A + BP_GROUP - 1) / BP_GROUP, tiles = bp_tiles(b.n), gz = (b.S + 3) / 4;
+    const int parts = std::min(groups, std::max(1, 2048 / (tiles * gz)));
+    const int per = (groups + parts - 1) / parts;
+    k.part = b.part;
+    k.per = per * BP_GROUP;
+    hipLaunchKernelGGL((k_backproject<float, 2, 16, 1, 1>), dim3(tiles, gz, (groups + per - 1) / per), dim3(256), 0, st, k);
+    RAFT_HIP(hipGetLastError());
+    const size_t count = (size_t)b.S * b.n * b.n;
+    hipLaunchKernelGGL(k_bp_groups, dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, st, b.part, b.out, groups, count);
+    RAFT_HIP(hipGetLastError());
+}
+
 int bp_tiles(int n) { return ((n + BP_TILE_X - 1) / BP_TILE_X) * ((n + BP_TILE_Y - 1) / BP_TILE_Y); }
 
 size_t bp_desc_size() { return sizeof(BpKArgs); }
@@ -605,6 +675,10 @@ void launch_backproject(const BpArgs& b, int store, hipStream_t st)
     }
     bp_check_rows(b, store);
     BpKArgs k = bp_kargs(b);
+    if (b.part && b.mode == 0) {
+        launch_backproject_split(b, k, st);
+        return;
+    }
     const int per = bp_slices_per_item(store, b.mode, b.chunk);
     const int groups = (b.S + per - 1) / per;
     if (groups > 65535) fail(RAFT_EUNSUPPORTED, "too many slice groups for one backprojection launch");

@@ -342,7 +342,7 @@ struct PinnedBuf {
 };
 
 struct Device {
-    static constexpr int kSlots = 15;
+    static constexpr int kSlots = 16;
     std::mutex mu;
     std::map<std::string, std::unique_ptr<FilterTables>> filters;
     DevBuf ws[kSlots];
@@ -654,6 +654,10 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
                                       t.chunk = c;
                                       launch_backproject(t, store, st);
                                   });
+        // few tiles: split over the angles (the tuned chunk then serves the calls
+        // that may not allocate)
+        const size_t split = mx ? 0 : bp_split_workspace(nb, N, A, store);
+        if (split && split <= budget / 4) ba.part = static_cast<float*>(D.workspace<15>(split));
         {
             ProfScope ps(KF_BP, st);
             launch_backproject(ba, store, st);

@@ -218,8 +218,11 @@ struct BpArgs {
     int chunk = 0;      // variant: angles per LDS round (16, 32 or 48; 0 = 32), | BP_PAIR for the pair form
     size_t q_bytes = 0; // bytes of the buffer behind q when known: launches that would read past it are refused
     const double* cs = nullptr; // matrix form: {cA, cB} pairs per angle
+    float* part = nullptr;      // FP32 rows, mode 0: workspace of the split form (bp_split_workspace)
 };
 void launch_backproject(const BpArgs& a, int store, hipStream_t st);
+// bytes of its workspace where few tiles should be split over the angles, else 0
+size_t bp_split_workspace(int S, int n, int A, int store);
 // whether an FBP call of S slices of n x n runs the matrix form (chunk =
 // BP_MX); decided once per call, so blocks of a call agree
 bool bp_matrix_form(int S, int n, int store);
