@@ -13,6 +13,9 @@
 // reads, zeros outside [0, n), into the slice-interleaved layout
 // [group][angle][bin][SB] (SB = 4 for FP32 rows, 8 for FP16 rows).
 //
+// Sizes of 64 M and 512 M bins run k_filter_dif instead: forward passes that
+// leave the spectrum permuted, H in that order, and the same passes back.
+//
 // Padded sizes with a prime factor > 5 or n > 16384 run the same circular
 // convolution q[m] = sum_j g[(m - j) mod n] u[j], g = IDFT(H) (built on the host
 // in FP64), in FP64: by transforms (k_filter_conv) or, for short rows and for
@@ -577,62 +580,111 @@ struct ConvK {
     unsigned rows; // (group, angle) pairs
 };
 
-__device__ __forceinline__ d2 zmul(d2 a, d2 b)
+template <typename V> __device__ __forceinline__ V zmul(V a, V b)
 {
-    return d2{fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
+    return V{fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
 }
-__device__ __forceinline__ d2 zconj(d2 a) { return d2{a.x, -a.y}; }
+template <typename V> __device__ __forceinline__ V zconj(V a) { return V{a.x, -a.y}; }
 // a * -i (forward), a * i (inverse)
-template <bool INV> __device__ __forceinline__ d2 zrot(d2 a) { return INV ? d2{-a.y, a.x} : d2{a.y, -a.x}; }
+template <bool INV, typename V> __device__ __forceinline__ V zrot(V a) { return INV ? V{-a.y, a.x} : V{a.y, -a.x}; }
 
-template <bool INV> __device__ __forceinline__ void zdft4(d2& a, d2& b, d2& c, d2& d)
+template <bool INV, typename V> __device__ __forceinline__ void zdft4(V& a, V& b, V& c, V& d)
 {
-    const d2 s = a + c, t = a - c, u = b + d, v = zrot<INV>(b - d);
+    const V s = a + c, t = a - c, u = b + d, v = zrot<INV>(b - d);
     a = s + u; b = t + v; c = s - u; d = t - v;
 }
-// DFT of v[0..R) in place, W = exp(-+ 2 pi i / R)
-template <int R, bool INV> __device__ __forceinline__ void zdft(d2 (&v)[R])
+
+// cos and sin of 2 pi m / R, by their series at compile time
+constexpr double series(double x, bool sine)
 {
-    static_assert(R == 3 || R == 4 || R == 5 || R == 8, "radix");
+    double term = sine ? x : 1.0, sum = term;
+    for (int k = sine ? 1 : 0; k < 40; k += 2) {
+        term *= -x * x / ((k + 1.0) * (k + 2.0));
+        sum += term;
+    }
+    return sum;
+}
+template <int R> struct Roots {
+    double c[R], s[R];
+    constexpr Roots() : c(), s()
+    {
+        for (int m = 0; m < R; ++m) {
+            const double x = 6.28318530717958647693 * (2 * m > R ? m - R : m) / R;
+            c[m] = series(x, false);
+            s[m] = series(x, true);
+        }
+    }
+};
+
+// DFT of v[0..R) in place, W = exp(-+ 2 pi i / R)
+template <int R, bool INV, typename V> __device__ __forceinline__ void zdft(V (&v)[R])
+{
+    using E = decltype(v[0].x + v[0].x);
     if constexpr (R == 3) {
-        const double h = 0.86602540378443864676; // sin 60 degrees
-        const d2 s = v[1] + v[2], m = v[0] - 0.5 * s, r = zrot<INV>(h * (v[1] - v[2]));
+        const E h = (E)0.86602540378443864676; // sin 60 degrees
+        const V s = v[1] + v[2], m = v[0] - (E)0.5 * s, r = zrot<INV>(h * (v[1] - v[2]));
         v[0] = v[0] + s; v[1] = m + r; v[2] = m - r;
+    } else if constexpr (R == 2) {
+        const V a = v[0], b = v[1];
+        v[0] = a + b; v[1] = a - b;
     } else if constexpr (R == 4) {
         zdft4<INV>(v[0], v[1], v[2], v[3]);
     } else if constexpr (R == 5) {
-        const double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410; // cos 72, cos 144 degrees
-        const double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;  // their sines
-        const d2 p1 = v[1] + v[4], p2 = v[2] + v[3], q1 = v[1] - v[4], q2 = v[2] - v[3];
-        const d2 m1 = v[0] + c1 * p1 + c2 * p2, m2 = v[0] + c2 * p1 + c1 * p2;
-        const d2 r1 = zrot<INV>(s1 * q1 + s2 * q2), r2 = zrot<INV>(s2 * q1 - s1 * q2);
+        const E c1 = (E)0.30901699437494742410, c2 = (E)-0.80901699437494742410; // cos 72, cos 144 degrees
+        const E s1 = (E)0.95105651629515357212, s2 = (E)0.58778525229247312917;  // their sines
+        const V p1 = v[1] + v[4], p2 = v[2] + v[3], q1 = v[1] - v[4], q2 = v[2] - v[3];
+        const V m1 = v[0] + c1 * p1 + c2 * p2, m2 = v[0] + c2 * p1 + c1 * p2;
+        const V r1 = zrot<INV>(s1 * q1 + s2 * q2), r2 = zrot<INV>(s2 * q1 - s1 * q2);
         v[0] = v[0] + p1 + p2;
         v[1] = m1 + r1; v[4] = m1 - r1; v[2] = m2 + r2; v[3] = m2 - r2;
-    } else {
-        const double h = 0.70710678118654752440; // sqrt(1/2)
+    } else if constexpr (R == 8) {
+        const E h = (E)0.70710678118654752440; // sqrt(1/2)
         zdft4<INV>(v[0], v[2], v[4], v[6]);
         zdft4<INV>(v[1], v[3], v[5], v[7]);
         // odd part times W_8^k, k = 0..3 (in v[1], v[3], v[5], v[7])
-        const d2 o1 = h * (v[3] + zrot<INV>(v[3])), o2 = zrot<INV>(v[5]), o3 = h * (zrot<INV>(v[7]) - v[7]);
-        const d2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
+        const V o1 = h * (v[3] + zrot<INV>(v[3])), o2 = zrot<INV>(v[5]), o3 = h * (zrot<INV>(v[7]) - v[7]);
+        const V e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
         v[0] = e0 + o0; v[4] = e0 - o0;
         v[1] = e1 + o1; v[5] = e1 - o1;
         v[2] = e2 + o2; v[6] = e2 - o2;
         v[3] = e3 + o3; v[7] = e3 - o3;
+    } else {
+        // R = A B: A-point transforms over n1 of v[B n1 + n2], W_R^(n2 k1), B-point
+        // transforms over n2
+        static_assert(R == 6 || R == 10 || R == 12 || R == 16, "radix");
+        constexpr int A = R == 6 ? 3 : (R == 10 ? 5 : 4), B = R / A;
+        constexpr Roots<R> W;
+        V t[B][A];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < A; ++n1) t[n2][n1] = v[B * n1 + n2];
+            zdft<A, INV>(t[n2]);
+#pragma unroll
+            for (int k1 = 1; k1 < A; ++k1)
+                if (n2 > 0) t[n2][k1] = zmul(t[n2][k1], V{(E)W.c[n2 * k1], (E)(INV ? W.s[n2 * k1] : -W.s[n2 * k1])});
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) {
+            V u[B];
+#pragma unroll
+            for (int n2 = 0; n2 < B; ++n2) u[n2] = t[n2][k1];
+            zdft<B, INV>(u);
+#pragma unroll
+            for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = u[k2];
+        }
     }
 }
-// v[q] *= W_len^(x q) (conjugate for the inverse)
-template <int R, bool INV> __device__ __forceinline__ void ztwiddle(d2 (&v)[R], const d2* tw, int x)
+// v[q] *= W_len^(x q) (conjugate for the inverse): the powers of two from the
+// table, the others their products
+template <int R, bool INV, typename V> __device__ __forceinline__ void ztwiddle(V (&v)[R], const V* tw, int x)
 {
-    d2 w[R];
-    w[1] = tw[x];
-    w[2] = tw[2 * x];
-    if constexpr (R > 4) w[4] = tw[4 * x];
-    if constexpr (R > 3) w[3] = zmul(w[1], w[2]);
-    if constexpr (R > 5) {
-        w[5] = zmul(w[1], w[4]);
-        w[6] = zmul(w[2], w[4]);
-        w[7] = zmul(w[3], w[4]);
+    V w[R];
+#pragma unroll
+    for (int q = 1; q < R; ++q) {
+        int top = 1;
+        while (2 * top <= q) top *= 2;
+        w[q] = q == top ? tw[q * x] : zmul(w[top], w[q - top]);
     }
 #pragma unroll
     for (int q = 1; q < R; ++q) v[q] = zmul(v[q], INV ? zconj(w[q]) : w[q]);
@@ -806,6 +858,225 @@ template <typename OT> void launch_conv(const FilterK& k, const FilterArgs& a, h
     RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_filter_conv<OT>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_filter_conv<OT>), dim3((unsigned)blocks), dim3(CV_THREADS), lds, st, k, c);
+}
+
+// ---- FP32 rows of n = M0 64 or M0 512 bins (k_filter_dif) -------------------
+//
+// The same passes in FP32 for the padded row itself (the circular convolution):
+// radix M0 from the sinogram, radix 8 in LDS down to blocks of 8, the product
+// with H (in the order that leaves) inside the last one, and back; the bins leave
+// from the registers of the last pass.  A workgroup takes two slice pairs of an
+// angle in turn and stores 16 bytes (FP16: 8) per bin; the first pair's window
+// waits in LDS.
+//
+// Why instead of the transforms in natural order (k_filter_fft*): LDS passes and
+// barriers bound those, and this form has 6 reads and 6 writes of LDS a pair
+// instead of 10 and 10 (n = 6144) and 12 barriers instead of about 24; its
+// twiddles come from tables in the lanes' order (products of two-level tables
+// before), so the rows' error is about half.  Filter time before -> now: 64 slices
+// of 2048 x 2048, n = 6144, FP32 rows in pieces 2.83 -> 1.64 ms, FP16 4.04 -> 1.52;
+// per row pair at n = 512 / 1024 / 2048 / 4096 / 6144 / 8192 3.5 / 7.2 / 13.7 / 27.5 /
+// 40.5 / 87.7 -> 1.7 / 3.5 / 9.2 / 20.7 / 28.0 / 51.0 ns.
+typedef float f2 __attribute__((ext_vector_type(2)));
+template <int M0, int E8> struct Dif {
+    static constexpr int M = E8 == 3 ? 512 : 64, LEN = M0 * M, TH = LEN / 8;
+    // waves per SIMD of as many workgroups as the LDS holds
+    static constexpr int WPE = TH > 768 ? 4 : (TH == 640 || (M0 == 16 && E8 == 2) ? 5 : 6); // the last: registers
+    static constexpr int PAD = LEN + LEN / 8 + 2; // complex values before the window
+};
+
+// v[q] *= W^(j q) (conjugate for the inverse) of a pass whose blocks have R M
+// elements, from its table [q][j < M] (neighbouring lanes, neighbouring
+// entries).  Powers below ONE and the multiples of ONE come from it, the others
+// are one product: the radix-8 passes take all seven (their tables stay in the
+// L1 cache; with products the error of the filtered rows grows by a fifth).
+template <int R, int M, bool INV, int ONE> __device__ __forceinline__ void dif_twiddle(f2 (&v)[R], const f2* tw, int j)
+{
+    f2 w[R];
+#pragma unroll
+    for (int q = 1; q < R; ++q)
+        w[q] = q < ONE || q % ONE == 0 ? tw[q * M + j] : zmul(w[q / ONE * ONE], w[q % ONE]);
+#pragma unroll
+    for (int q = 1; q < R; ++q) v[q] = zmul(v[q], INV ? zconj(w[q]) : w[q]);
+}
+
+template <int LEN, int TH, int B, bool INV> __device__ __forceinline__ void dif_pass(f2* z, const f2* tw, int b)
+{
+    constexpr int M = B / 8;
+    const int j = b & (M - 1), base = (b / M) * B + j; // one butterfly a thread
+    f2 v[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = z[cpix(base + t * M)];
+    if (INV) dif_twiddle<8, M, true, 8>(v, tw, j);
+    zdft<8, INV>(v);
+    if (!INV) dif_twiddle<8, M, false, 8>(v, tw, j);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) z[cpix(base + t * M)] = v[t];
+}
+
+template <typename OT, int M0, int E8, bool ROWS>
+__global__ __launch_bounds__((Dif<M0, E8>::TH), (Dif<M0, E8>::WPE)) void k_filter_dif(FilterK a, const f2* __restrict__ H,
+                                                                                   const f2* __restrict__ tw, unsigned rows)
+{
+    using D = Dif<M0, E8>;
+    constexpr int M = D::M, TH = D::TH, LEN = D::LEN;
+    constexpr bool F32 = sizeof(OT) == 4;
+    extern __shared__ __align__(16) char conv_smem[];
+    f2* z = reinterpret_cast<f2*>(conv_smem);
+    f2* win = z + D::PAD;                         // [W]: the first pair's window (FP16: packed)
+    unsigned* winh = reinterpret_cast<unsigned*>(win);
+    // the halves of an FP16 entry on one XCD (see k_filter_conv)
+    constexpr unsigned per = F32 ? 1 : 2;
+    const unsigned ga = (blockIdx.x >> 3) / per * 8u + (blockIdx.x & 7u);
+    if (ga >= rows) return;
+    const int ang = (int)(ga % (unsigned)a.A), g = (int)(ga / (unsigned)a.A);
+    const int s0 = g * a.SB + 4 * (int)((blockIdx.x >> 3) % per); // first of the four slices
+    const float wv = a.wa[ang];
+    const size_t ri = row_index(a, g, ang);
+    const size_t ss = (size_t)a.A * a.N;
+
+    auto store = [&](int w, f2 lo, f2 hi) __attribute__((always_inline)) {
+        if constexpr (ROWS) {
+            // the group's four rows of this angle, each written by this workgroup
+            // only and after all of them were read (in place when rows is tomo)
+            float* r = a.rows + ((size_t)s0 * a.A + ang) * a.W + w;
+            const size_t rs = (size_t)a.A * a.W;
+            if (s0 < a.S) r[0] = lo.x;
+            if (s0 + 1 < a.S) r[rs] = lo.y;
+            if (s0 + 2 < a.S) r[2 * rs] = hi.x;
+            if (s0 + 3 < a.S) r[3 * rs] = hi.y;
+        } else if constexpr (F32) {
+            store_entry(a, ri, w, make_float4(lo.x, lo.y, hi.x, hi.y));
+        } else {
+            const __half2 h0 = __floats2half2_rn(lo.x, lo.y), h1 = __floats2half2_rn(hi.x, hi.y);
+            reinterpret_cast<uint2*>(a.q)[(ri * a.W + w) * 2 + (s0 - g * a.SB) / 4] =
+                make_uint2(*reinterpret_cast<const unsigned*>(&h0), *reinterpret_cast<const unsigned*>(&h1));
+        }
+    };
+    // bins outside [0, n) are zero
+    for (int w = threadIdx.x; w < a.W; w += TH)
+        if (a.tlo + w < 0 || a.tlo + w >= LEN) store(w, f2{0.0f, 0.0f}, f2{0.0f, 0.0f});
+
+#pragma unroll 1
+    for (int pr = 0; pr < 2; ++pr) {
+        // opaque: what depends on it (twiddles, addresses) is formed where it is
+        // used, not kept in registers across the pairs
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int sl = s0 + 2 * pr;
+        const bool h0 = sl < a.S, h1 = sl + 1 < a.S; // missing slices are zero
+        const float* r0 = a.tomo + ((size_t)sl * a.A + ang) * a.N;
+        for (int j = tid; j < M; j += TH) {
+            f2 v[M0];
+#pragma unroll
+            for (int t = 0; t < M0; ++t) {
+                const int i = min(max(j + t * M - a.L, 0), a.N - 1);
+                v[t] = f2{h0 ? r0[i] : 0.0f, h1 ? r0[ss + i] : 0.0f};
+            }
+            zdft<M0, false>(v);
+            dif_twiddle<M0, M, false, 4>(v, tw, j);
+#pragma unroll
+            for (int t = 0; t < M0; ++t) z[cpix(j + t * M)] = v[t];
+        }
+        __syncthreads();
+        if constexpr (E8 == 3) {
+            dif_pass<LEN, TH, 512, false>(z, tw + LEN, tid);
+            __syncthreads();
+        }
+        dif_pass<LEN, TH, 64, false>(z, tw + LEN + 512, tid);
+        __syncthreads();
+        {
+            const int b = 8 * tid;
+            f2 v[8], h[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) h[t] = H[b + t];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = z[cpix(b) + t];
+            zdft<8, false>(v);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = zmul(v[t], h[t]);
+            zdft<8, true>(v);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) z[cpix(b) + t] = v[t];
+        }
+        __syncthreads();
+        dif_pass<LEN, TH, 64, true>(z, tw + LEN + 512, tid);
+        __syncthreads();
+        if constexpr (E8 == 3) {
+            dif_pass<LEN, TH, 512, true>(z, tw + LEN, tid);
+            __syncthreads();
+        }
+        for (int j = tid; j < M; j += TH) {
+            f2 v[M0];
+#pragma unroll
+            for (int t = 0; t < M0; ++t) v[t] = z[cpix(j + t * M)];
+            dif_twiddle<M0, M, true, 4>(v, tw, j);
+            zdft<M0, true>(v);
+#pragma unroll
+            for (int t = 0; t < M0; ++t) {
+                const int w = j + t * M - a.tlo;
+                if ((unsigned)w >= (unsigned)a.W) continue;
+                const f2 x = v[t] * wv;
+                if (pr == 0) {
+                    // read back by the same thread
+                    if constexpr (F32) {
+                        win[w] = x;
+                    } else {
+                        const __half2 hx = __floats2half2_rn(x.x, x.y);
+                        winh[w] = *reinterpret_cast<const unsigned*>(&hx);
+                    }
+                } else if constexpr (F32) {
+                    store(w, win[w], x);
+                } else {
+                    const __half2 hx = __floats2half2_rn(x.x, x.y);
+                    reinterpret_cast<uint2*>(a.q)[(ri * a.W + w) * 2 + (s0 - g * a.SB) / 4] =
+                        make_uint2(winh[w], *reinterpret_cast<const unsigned*>(&hx));
+                }
+            }
+        }
+        if (pr == 0) __syncthreads(); // the row is read before the next overwrites it
+    }
+}
+
+template <typename OT, int M0, int E8> bool launch_dif_t(const FilterK& k, const FilterArgs& a, hipStream_t st)
+{
+    using D = Dif<M0, E8>;
+    const size_t lds = sizeof(float2) * D::PAD + (size_t)k.W * (sizeof(OT) == 4 ? 8 : 4);
+    if (lds > 160 * 1024) return false;
+    const unsigned rows = (unsigned)((long long)((k.S + k.SB - 1) / k.SB) * k.A);
+    const long long blocks = ((long long)rows + 7) / 8 * 8 * (k.SB / 4);
+    if (blocks > 0x7fffffffLL) return false;
+    const f2* H = reinterpret_cast<const f2*>(a.dif_H);
+    const f2* tw = reinterpret_cast<const f2*>(a.dif_tw);
+    const bool direct = sizeof(OT) == 4 && k.rows;
+    const void* fn = reinterpret_cast<const void*>(&k_filter_dif<OT, M0, E8, false>);
+    if constexpr (sizeof(OT) == 4)
+        if (direct) fn = reinterpret_cast<const void*>(&k_filter_dif<OT, M0, E8, true>);
+    RAFT_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    FilterK kk = k;
+    unsigned rr = rows;
+    void* args[] = {&kk, &H, &tw, &rr};
+    RAFT_HIP(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(D::TH), args, lds, st));
+    return true;
+}
+// false: not a size of this form
+template <typename OT> bool launch_dif(const FilterK& k, const FilterArgs& a, hipStream_t st)
+{
+    switch (k.npad) {
+    case 512: return launch_dif_t<OT, 8, 2>(k, a, st);
+    case 640: return launch_dif_t<OT, 10, 2>(k, a, st);
+    case 768: return launch_dif_t<OT, 12, 2>(k, a, st);
+    case 1024: return launch_dif_t<OT, 16, 2>(k, a, st);
+    case 1536: return launch_dif_t<OT, 3, 3>(k, a, st);
+    case 2048: return launch_dif_t<OT, 4, 3>(k, a, st);
+    case 2560: return launch_dif_t<OT, 5, 3>(k, a, st);
+    case 3072: return launch_dif_t<OT, 6, 3>(k, a, st);
+    case 4096: return launch_dif_t<OT, 8, 3>(k, a, st);
+    case 5120: return launch_dif_t<OT, 10, 3>(k, a, st);
+    case 6144: return launch_dif_t<OT, 12, 3>(k, a, st);
+    case 8192: return launch_dif_t<OT, 16, 3>(k, a, st);
+    default: return false;
+    }
 }
 
 template <typename OT, int THREADS, int E>
@@ -1310,6 +1581,52 @@ FftPlan fft_plan(int n)
     return p;
 }
 
+// first radix of the FP32 form (k_filter_dif), 0: none
+static int dif_radix(int n)
+{
+    for (int m : {8, 10, 12, 16})
+        if (n == 64 * m) return m;
+    for (int m : {3, 4, 5, 6, 8, 10, 12, 16})
+        if (n == 512 * m) return m;
+    return 0;
+}
+
+// frequency held at each position after forward passes of these radices:
+// position q (block / radix) + r holds radix f(r) + q
+static std::vector<int> dif_order(const int* radix, int passes)
+{
+    std::vector<int> freq(1, 0);
+    for (int i = passes - 1; i >= 0; --i) {
+        std::vector<int> up;
+        for (int q = 0; q < radix[i]; ++q)
+            for (int f : freq) up.push_back(radix[i] * f + q);
+        freq.swap(up);
+    }
+    return freq;
+}
+
+bool dif_tables(int n, const std::vector<float2>& H, std::vector<float2>& Hp, std::vector<float2>& tw)
+{
+    const int m = dif_radix(n);
+    if (!m) return false;
+    const int radix[4] = {m, 8, 8, 8};
+    const std::vector<int> freq = dif_order(radix, n == 64 * m ? 3 : 4);
+    Hp.resize(n);
+    for (int e = 0; e < n; ++e) Hp[e] = H[freq[e]];
+    // exp(-2 pi i q j / (R M)), [q < R][j < M], of the first pass and of the
+    // radix-8 passes over blocks of 512 and 64
+    tw.clear();
+    for (int R : {m, 8, 8}) {
+        const int M = tw.empty() ? n / m : (tw.size() == (size_t)n ? 64 : 8);
+        for (int q = 0; q < R; ++q)
+            for (int j = 0; j < M; ++j) {
+                const double ang = -2.0 * M_PI * (double)q * (double)j / ((double)R * M);
+                tw.push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
+            }
+    }
+    return true;
+}
+
 ConvPlan conv_plan(int n, int N)
 {
     ConvPlan best;
@@ -1343,15 +1660,7 @@ void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::v
         w[2 * k] = std::cos(ang);
         w[2 * k + 1] = std::sin(ang);
     }
-    // frequency held at each position after the forward passes: position
-    // q (block / radix) + r holds radix f(r) + q
-    std::vector<int> freq(1, 0);
-    for (int i = p.passes - 1; i >= 0; --i) {
-        std::vector<int> up;
-        for (int q = 0; q < p.radix[i]; ++q)
-            for (int f : freq) up.push_back(p.radix[i] * f + q);
-        freq.swap(up);
-    }
+    const std::vector<int> freq = dif_order(p.radix, p.passes);
     spec.assign(2 * (size_t)len * p.chunks, 0.0);
     std::vector<double> x(2 * (size_t)len), y(2 * (size_t)len);
     for (int c = 0; c < p.chunks; ++c) {
@@ -1422,7 +1731,14 @@ bool launch_fbp_filter(const FilterArgs& a, const FftPlan& plan, int store, hipS
     if (blocks > 0x7fffffffLL) fail(RAFT_EUNSUPPORTED, "too many sinogram rows for one filter launch");
     const size_t lds = sizeof(float2) * lds_elems(a.npad);
     const size_t lds_fft = lds + sizeof(float2) * (size_t)(128 + a.npad / 128 + 1);
-    if (plan.ok || a.none) {
+    bool done = false;
+    if (a.dif_H && !a.none) {
+        if (store == RAFT_STORE_F16) done = launch_dif<__half>(k, a, st);
+        else done = launch_dif<float>(k, a, st);
+        direct = done && k.rows != nullptr;
+    }
+    if (done) {
+    } else if (plan.ok || a.none) {
         const FftK p = fftk_of(plan);
         const int threads = plan.ok ? plan.threads : 256;
         if (store == RAFT_STORE_F16) launch_fft<__half>(k, p, threads, (int)blocks, lds_fft, st);

@@ -297,6 +297,7 @@ static double filter_apply(int type, double w, double reg, double pag)
 struct FilterTables {
     DevBuf H, tw, g; // float2[n], float2[n], double[n]
     DevBuf spec, ctw, edge; // see conv_tables
+    DevBuf difH, diftw;     // see dif_tables
     FftPlan plan;
     ConvPlan conv;
     void set(FilterArgs& a) const
@@ -308,6 +309,8 @@ struct FilterTables {
         a.conv_spec = spec.p;
         a.conv_tw = ctw.p;
         a.conv_edge = static_cast<const double*>(edge.p);
+        a.dif_H = static_cast<const float2*>(difH.p);
+        a.dif_tw = static_cast<const float2*>(diftw.p);
     }
 };
 
@@ -458,7 +461,7 @@ template <typename T> static void upload(DevBuf& b, const std::vector<T>& v, hip
 // 1/(npad*pixel)), the FFT twiddles and, for sizes the LDS FFT does not take,
 // the real convolution kernel g
 struct FilterHost {
-    std::vector<float2> H, tw;
+    std::vector<float2> H, tw, difH, diftw;
     std::vector<double> g, spec, ctw, edge;
     FftPlan plan;
     ConvPlan conv;
@@ -495,6 +498,7 @@ static void filter_host_tables(const FbpCfg& c, FilterHost& F)
         F.tw[128 + k] = make_float2((float)std::cos(ang), (float)std::sin(ang));
     }
     F.plan = fft_plan(n);
+    dif_tables(n, F.H, F.difH, F.diftw);
     F.g.clear();
     if (!F.plan.ok && c.filter != 0) {
         // g[d] = sum_k H_k exp(2 pi i k d / n): real because H is Hermitian
@@ -535,6 +539,10 @@ static FilterTables& filter_tables(Device& D, const FbpCfg& c, hipStream_t st)
     upload(F->H, h.H, st);
     upload(F->tw, h.tw, st);
     if (!h.g.empty()) upload(F->g, h.g, st);
+    if (!h.difH.empty()) {
+        upload(F->difH, h.difH, st);
+        upload(F->diftw, h.diftw, st);
+    }
     F->conv = h.conv;
     if (h.conv.len) {
         upload(F->spec, h.spec, st);
@@ -730,13 +738,17 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     const size_t oH = put(F->H.data(), F->H.size() * sizeof(float2));
     const size_t oTw = put(F->tw.data(), F->tw.size() * sizeof(float2));
     const size_t oG = put(F->g.data(), F->g.size() * sizeof(double));
-    // the convolution form's tables, where a slice group of rows still fits
-    // behind them (else the direct sum of the same FP64 terms)
+    // the tables of the faster filter forms, where a slice group of rows still
+    // fits behind them (else the general forms: the same sums, rounded apart)
     const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
     const size_t per_group = (size_t)A * g.width * 16;
     const size_t cap = (size_t)RAFT_NOALLOC_SCRATCH_BYTES;
     const size_t conv_bytes = (F->spec.size() + F->ctw.size() + F->edge.size()) * sizeof(double) + 3 * 256;
     const bool conv = F->conv.len > 0 && host.size() + conv_bytes + (size_t)A * 20 + 4 * 256 + per_group <= cap;
+    const bool dif = !F->difH.empty() &&
+                     host.size() + (F->difH.size() + F->diftw.size()) * sizeof(float2) + (size_t)A * 20 + 7 * 256 + per_group <= cap;
+    const size_t oDifH = dif ? put(F->difH.data(), F->difH.size() * sizeof(float2)) : 0;
+    const size_t oDifTw = dif ? put(F->diftw.data(), F->diftw.size() * sizeof(float2)) : 0;
     const size_t oSpec = conv ? put(F->spec.data(), F->spec.size() * sizeof(double)) : 0;
     const size_t oCtw = conv ? put(F->ctw.data(), F->ctw.size() * sizeof(double)) : 0;
     const size_t oEdge = conv ? put(F->edge.data(), F->edge.size() * sizeof(double)) : 0;
@@ -791,6 +803,10 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
             fa.conv_spec = base + oSpec;
             fa.conv_tw = base + oCtw;
             fa.conv_edge = reinterpret_cast<const double*>(base + oEdge);
+        }
+        if (dif) {
+            fa.dif_H = reinterpret_cast<const float2*>(base + oDifH);
+            fa.dif_tw = reinterpret_cast<const float2*>(base + oDifTw);
         }
         fa.wa = reinterpret_cast<const float*>(base + oW);
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = g.tlo; fa.W = g.width;

@@ -161,6 +161,10 @@ ConvPlan conv_plan(int n, int N);
 void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::vector<double>& spec,
                  std::vector<double>& tw, std::vector<double>& edge);
 
+// tables of the FP32 form for sizes that have it (false: none): H in the order
+// its forward passes leave, and the passes' twiddles
+bool dif_tables(int n, const std::vector<float2>& H, std::vector<float2>& Hp, std::vector<float2>& tw);
+
 struct FilterArgs {
     const float* tomo;  // [S][A][N]
     void* q;            // [G][A][W][SB] float (SB = 4) or __half (SB = 8)
@@ -171,6 +175,8 @@ struct FilterArgs {
     const void* conv_spec = nullptr;
     const void* conv_tw = nullptr;
     const double* conv_edge = nullptr;
+    const float2* dif_H = nullptr; // with dif_tw (see dif_tables) or null
+    const float2* dif_tw = nullptr;
     const float* wa;    // [A] per-angle weight (dtheta * angular scale)
     int N, A, S, npad, L, tlo, W;
     int none;           // filter 'none': no filtering, no 1/(npad h)
