@@ -190,11 +190,12 @@ __device__ __forceinline__ void fft_pass(float2* z, const Tw& tw, int n, int Ns,
     __syncthreads();
 }
 
-// Waves per SIMD asked of the 768-thread LDS FFT kernels (n in (4096, 6144]):
-// six keep them within 80 VGPRs, so two workgroups share a CU (twice ~54 KB
-// of LDS at n = 6144) and one workgroup's barriers overlap the other's passes.
-// Other sizes fit several workgroups per CU at their natural register count.
-template <int THREADS> constexpr int fft_wpe() { return THREADS == 768 ? 6 : 1; }
+// Waves per SIMD asked of the LDS FFT kernels: six keep them within 80 VGPRs, so
+// that as many workgroups share a CU as their LDS allows (768 threads, n in
+// (4096, 6144]: two instead of one; 384 threads: four instead of three) and one
+// workgroup's barriers overlap the others' passes.  16 slices, n = 3072: the polar
+// pass 0.51 -> 0.44 ms, the second inverse transform 0.37 -> 0.31.
+template <int THREADS> constexpr int fft_wpe() { return THREADS <= 768 ? 6 : 1; }
 
 struct FftK {
     int n, nstages;
@@ -1361,6 +1362,10 @@ __global__ void k_bst_p2c(const float2* polar, float2* cart, int n, int A2, int 
 // [L, L + N) the crop keeps are written, as rows of out [S][s][N].  The grid
 // is never written to HBM.  The expressions are those of the two unfused
 // kernels, so the values are the same bit for bit.
+// Waiting for the gathers and between the passes bounds it, so what counts is
+// workgroups per CU: the cells' derived values are formed in each slice's turn
+// (kept for all cells across the slices they took 163 registers: two workgroups
+// of 384 threads; 112 now).  16 slices of 3072 x 3072 cells: 1.76 -> 1.23 ms.
 constexpr int BST_SPB = 8;
 struct BstRowsK {
     const float2* polar; // [S][A2][n/2]
@@ -1369,7 +1374,7 @@ struct BstRowsK {
 };
 
 template <int THREADS, int E, int EC>
-__global__ __launch_bounds__(THREADS) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
+__global__ __launch_bounds__(THREADS, 4) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
 {
     extern __shared__ float2 z[];
     const int n = a.n, s = a.s;
@@ -1377,7 +1382,10 @@ __global__ __launch_bounds__(THREADS) void k_bst_rows(BstRowsK a, const float2* 
     const int ntw = 128 + n / 128 + 1;
     for (int k = threadIdx.x; k < ntw; k += THREADS) tws[k] = twg[k];
     const Tw tw{tws, tws + 128};
-    const int tyd = blockIdx.x;
+    // runs of 8 neighbouring rows on one XCD (workgroups go to the 8 XCDs round
+    // robin): their cells share lines of the polar rows
+    const int tyd = (int)(blockIdx.x / 64u * 64u + (blockIdx.x & 7u) * 8u + (blockIdx.x >> 3) % 8u);
+    if (tyd >= s) return;
     const int sl0 = blockIdx.y * BST_SPB, sl1 = min(a.S, sl0 + BST_SPB);
     const int ty = (tyd + s - s / 2) % s; // (ty + s/2) % s == tyd
     // the cells txd = threadIdx.x + j THREADS of this row (THREADS EC >= s), in
@@ -1412,17 +1420,23 @@ __global__ __launch_bounds__(THREADS) void k_bst_rows(BstRowsK a, const float2* 
     }
     for (int sl = sl0; sl < sl1; ++sl) {
         const float2* P = a.polar + (size_t)sl * a.A2 * h;
+        // opaque: what depends on the cells is formed in each slice's turn, not
+        // kept in registers for all cells
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
         __syncthreads(); // the previous slice's row is read (and the twiddles are in)
 #pragma unroll
         for (int j = 0; j < EC; ++j) {
-            const int txd = threadIdx.x + j * THREADS;
+            const int txd = tid + j * THREADS;
+            int o = oc[j];
+            float pj = ps[j], tfrac = tf[j];
+            asm volatile("" : "+v"(o), "+v"(pj), "+v"(tfrac));
             if (txd < s) {
                 float2 val = make_float2(0.0f, 0.0f);
-                const float pfrac = fabsf(ps[j]);
-                if (oc[j] >= 0) {
-                    const int o0 = oc[j] & ((1 << 30) - 1);
-                    const int o1 = (oc[j] >> 30) ? o0 - wrapb : o0 + h;
-                    const float tfrac = tf[j];
+                const float pfrac = fabsf(pj);
+                if (o >= 0) {
+                    const int o0 = o & ((1 << 30) - 1);
+                    const int o1 = (o >> 30) ? o0 - wrapb : o0 + h;
                     const float2 a0 = P[o0], a1 = P[o0 + 1];
                     const float2 b0 = P[o1], b1 = P[o1 + 1];
                     const float2 i0 = make_float2(a0.x * (1.0f - pfrac) + a1.x * pfrac,
@@ -1431,14 +1445,14 @@ __global__ __launch_bounds__(THREADS) void k_bst_rows(BstRowsK a, const float2* 
                                                   b0.y * (1.0f - pfrac) + b1.y * pfrac);
                     val = make_float2(i0.x * tfrac + i1.x * (1.0f - tfrac), i0.y * tfrac + i1.y * (1.0f - tfrac));
                 }
-                const float sg = __builtin_signbit(ps[j]) ? -1.0f : 1.0f;
+                const float sg = __builtin_signbit(pj) ? -1.0f : 1.0f;
                 const float2 v = make_float2(val.x * sg, val.y * sg);
                 z[pix(txd)] = make_float2(v.x, -v.y);
             }
         }
         __syncthreads();
-        fft_run<THREADS, E>(z, tw, p);
-        for (int c = threadIdx.x; c < a.N; c += THREADS) {
+        fft_run<THREADS, E>(z, tw, p, tid);
+        for (int c = tid; c < a.N; c += THREADS) {
             const float2 v = z[pix(a.L + c)];
             a.out[((size_t)sl * s + tyd) * a.N + c] = make_float2(v.x, -v.y);
         }
@@ -1502,7 +1516,7 @@ void launch_bst_rows_t(const BstRowsK& k, const float2* tw, const FftK& p, size_
 {
     RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bst_rows<THREADS, E, EC>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_bst_rows<THREADS, E, EC>), dim3((unsigned)k.s, (unsigned)((k.S + BST_SPB - 1) / BST_SPB)),
+    hipLaunchKernelGGL((k_bst_rows<THREADS, E, EC>), dim3((unsigned)(k.s + 63) / 64u * 64u, (unsigned)((k.S + BST_SPB - 1) / BST_SPB)),
                        dim3(THREADS), lds, st, k, tw, p);
 }
 
