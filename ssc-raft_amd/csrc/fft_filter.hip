@@ -193,9 +193,10 @@ __device__ __forceinline__ void fft_pass(float2* z, const Tw& tw, int n, int Ns,
 // Waves per SIMD asked of the LDS FFT kernels: six keep them within 80 VGPRs, so
 // that as many workgroups share a CU as their LDS allows (768 threads, n in
 // (4096, 6144]: two instead of one; 384 threads: four instead of three) and one
-// workgroup's barriers overlap the others' passes.  16 slices, n = 3072: the polar
+// workgroup's barriers overlap the others' passes (shorter rows: their calls are
+// mostly too small to fill the chip).  16 slices, n = 3072: the polar
 // pass 0.51 -> 0.44 ms, the second inverse transform 0.37 -> 0.31.
-template <int THREADS> constexpr int fft_wpe() { return THREADS <= 768 ? 6 : 1; }
+template <int THREADS> constexpr int fft_wpe() { return THREADS >= 384 && THREADS <= 768 ? 6 : 1; }
 
 struct FftK {
     int n, nstages;
@@ -1366,6 +1367,8 @@ __global__ void k_bst_p2c(const float2* polar, float2* cart, int n, int A2, int 
 // workgroups per CU: the cells' derived values are formed in each slice's turn
 // (kept for all cells across the slices they took 163 registers: two workgroups
 // of 384 threads; 112 now).  16 slices of 3072 x 3072 cells: 1.76 -> 1.23 ms.
+// Below 256 threads few workgroups run at all and keeping the values is faster
+// (16 slices of 600 x 600: 34 us against 37).
 constexpr int BST_SPB = 8;
 struct BstRowsK {
     const float2* polar; // [S][A2][n/2]
@@ -1374,8 +1377,9 @@ struct BstRowsK {
 };
 
 template <int THREADS, int E, int EC>
-__global__ __launch_bounds__(THREADS, 4) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
+__global__ __launch_bounds__(THREADS, THREADS >= 256 ? 4 : 1) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
 {
+    constexpr bool BY_SLICE = THREADS >= 256;
     extern __shared__ float2 z[];
     const int n = a.n, s = a.s;
     float2* tws = z + lds_elems(n);
@@ -1423,14 +1427,14 @@ __global__ __launch_bounds__(THREADS, 4) void k_bst_rows(BstRowsK a, const float
         // opaque: what depends on the cells is formed in each slice's turn, not
         // kept in registers for all cells
         int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
+        if (BY_SLICE) asm volatile("" : "+v"(tid));
         __syncthreads(); // the previous slice's row is read (and the twiddles are in)
 #pragma unroll
         for (int j = 0; j < EC; ++j) {
             const int txd = tid + j * THREADS;
             int o = oc[j];
             float pj = ps[j], tfrac = tf[j];
-            asm volatile("" : "+v"(o), "+v"(pj), "+v"(tfrac));
+            if (BY_SLICE) asm volatile("" : "+v"(o), "+v"(pj), "+v"(tfrac));
             if (txd < s) {
                 float2 val = make_float2(0.0f, 0.0f);
                 const float pfrac = fabsf(pj);
