@@ -1367,8 +1367,10 @@ __global__ void k_bst_p2c(const float2* polar, float2* cart, int n, int A2, int 
 // workgroups per CU: the cells' derived values are formed in each slice's turn
 // (kept for all cells across the slices they took 163 registers: two workgroups
 // of 384 threads; 112 now).  16 slices of 3072 x 3072 cells: 1.76 -> 1.23 ms.
-// Below 256 threads few workgroups run at all and keeping the values is faster
-// (16 slices of 600 x 600: 34 us against 37).
+// 768 threads are held to 80 registers (some spill): two workgroups on a CU
+// instead of one, 8 slices of 6144 x 6144 cells, the call 3.26 -> 3.16 ms (3.40 with
+// one).  Below 256 threads few workgroups run at all and keeping the values is
+// faster (16 slices of 600 x 600: 34 us against 37).
 constexpr int BST_SPB = 8;
 struct BstRowsK {
     const float2* polar; // [S][A2][n/2]
@@ -1377,7 +1379,7 @@ struct BstRowsK {
 };
 
 template <int THREADS, int E, int EC>
-__global__ __launch_bounds__(THREADS, THREADS >= 256 ? 4 : 1) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
+__global__ __launch_bounds__(THREADS, THREADS == 768 ? 6 : (THREADS >= 256 ? 4 : 1)) void k_bst_rows(BstRowsK a, const float2* twg, FftK p)
 {
     constexpr bool BY_SLICE = THREADS >= 256;
     extern __shared__ float2 z[];
