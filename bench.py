@@ -7,15 +7,16 @@ sinogram (Poisson, I0 = 1e4) already resident in HBM.  One step = one
 raft_fbp_device call over the 64 slices (pad + FFT filter + backprojection).
 
 Also reported on the same JSON line:
-  roofline      backprojection kernel (k_backproject<float,0>): bound "valu",
+  roofline      backprojection kernel (k_backproject_mx<0>): bound "valu",
                 2 FLOP per gathered sample over its average launch time (HIP
                 events on the launch stream) against the 157.3 TFLOP/s FP32
                 vector peak; beside it the effective gather bandwidth, the
                 measured HBM traffic and its fraction of 8 TB/s, the
-                counter VALU issue rate (profiles/), and `lds`: the gathers'
-                LDS read bytes (4 per sample) over the launch time against
-                the device's conflict-free LDS read rate measured at start-up
-                by raft_lds_read_probe (the binding limit of the FP32 rows);
+                counter VALU issue rate (profiles/), and `lds`: the kernel's
+                LDS read bytes (the matrix operands: 1.6 per sample; the
+                projectors' gathers: 4) over the launch time against the
+                device's conflict-free LDS read rate measured at start-up by
+                raft_lds_read_probe;
   cpu_baseline  the FP32 restatement in oracle/ timed on this host's cores on
                 a bounded sample (whole slices of the same workload);
   fp16_rows     the same FBP with FP16-stored filtered rows;
@@ -297,10 +298,12 @@ def fbp_bench(args, torch, dv, ph):
     samples = float(S) * A * N * N
     bytes_alg = samples * 4 + float(S) * A * width * 4 + float(S) * N * N * 4
     bp_s = res["f32"]["bp_ms"] * 1e-3
-    roof = valu_roofline("k_backproject<float,0>", samples, bp_s, bytes_alg,
+    # LDS: three operands of 2 KB per 30 pixels x 4 angles x 32 slices
+    roof = valu_roofline("k_backproject_mx<0>", samples, bp_s, bytes_alg,
                          traffic=read_traffic("fbp_backproject_2048_traffic.txt"),
                          valu_issue=read_profile_value("backproject_projector_counters.txt",
-                                                       "valu_issue.k_backproject<float,0>"))
+                                                       "valu_issue.k_backproject_mx<0>"),
+                         lds_bytes_per_sample=3 * 2048 / (30 * 4 * 32))
     roof.update(gathered_bytes_per_launch=bytes_alg, staged_row_width=width, fft_path=bool(fft_path))
     return res, roof, cpu, radon, pcie
 

@@ -96,9 +96,11 @@ int raft_fbp_device(int device, float* d_obj, const float* d_tomo, const float* 
 /* raft_fbp_device that allocates no device memory.  No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * arguments, same kernels and the same output bit for bit (where the array
- * holds fewer than 16 slices, a call that raft_fbp_device sums on the matrix
- * cores keeps the gather kernels here and differs by rounding); the filter and
+ * arguments, same kernels and the same output bit for bit, but for two cases
+ * that differ by rounding: where the array holds fewer than 16 slices, a call
+ * that raft_fbp_device sums on the matrix cores keeps the gather kernels here;
+ * where one slice group fits only without the faster filter forms' tables, the
+ * general ones run.  The filter and
  * angle tables and the filtered rows live in one fixed device array of
  * RAFT_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
  * process ends, and the slices run in blocks of as many slice groups (4 slices
