@@ -356,7 +356,7 @@ __global__ __launch_bounds__(64 * PROJ_ANGLES, 4) void k_project(ProjK a)
 // Rays of a tile: the sampling grid is a rotation (ry rx = 1), so ray index is
 // affine in the pixel; the rays within `half` of the tile's centre hold all its
 // samples (margins of 1.5 pixels, as truncation takes (-1, 0) to pixel 0), and
-// both kernels number them from pt_first.  Samples are taken from a generous
+// both kernels number them from TileRays::first.  Samples are taken from a generous
 // range of k and tested exactly, in integers, against the tile.
 //
 // A wave's lane takes ray lane / 4 of 16 neighbouring ones and every fourth
@@ -365,7 +365,8 @@ __global__ __launch_bounds__(64 * PROJ_ANGLES, 4) void k_project(ProjK a)
 //
 // What bounds it: vector operations, twelve for a sample's place (five in FP64)
 // and four for its sums.  Two slice groups share the places where there are two
-// (their rows side by side; 16 waves, 136 KB, one workgroup per CU; one group: 8 waves, two workgroups).
+// (their rows side by side; 16 waves, 136 KB, one workgroup per CU; one group: 8
+// waves, two workgroups).
 // Tiles of 64 keep the partial sums at 1.3 / 64 of the samples.
 //
 // Projection, direct form -> this one: 6 slices of 700 x 500, 90 angles 0.76 ->
@@ -1108,6 +1109,7 @@ static void launch_tiles(const ProjArgs& p, const ProjK& k, int em_mode, int G, 
     } else if (gc < G) {
         gc &= ~1; // pairs of groups
     }
+    ac = std::min(ac, 65535); // k_project_sum: one grid row per angle
     const int tiles = t.tx * t.ty;
     for (t.g0 = 0; t.g0 < G; t.g0 += gc)
         for (t.a0 = 0; t.a0 < k.nangles; t.a0 += ac) {
