@@ -26,7 +26,7 @@ def _angles(a, first=0.0):
     (190, 130, 150, 30, 7, 1.0, 0.7),
     (100, 140, 100, 11, 3, 0.5, 1.0),
     (700, 500, 700, 90, 6, 1.0, 1.0),    # two slice groups a workgroup
-    (2048, 2048, 2048, 100, 8, 1.0, 1.0),  # angles in turns
+    (2048, 2048, 2048, 200, 8, 1.0, 1.0),  # angles in turns
 ])
 def test_radon_tiles_match_direct(gpu, monkeypatch, nx, ny, r, a, s, ax, ay):
     import torch
