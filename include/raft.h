@@ -221,11 +221,19 @@ int raft_eem_kl_device(int device, const float* d_obj, const float* d_tomo, cons
                        double* kl, long long* kl_excluded, void* stream);
 
 /* Host-only planning query (no device work): the bin window the FBP
- * backprojector stages per angle row for these parameters -- first bin *tlo
- * and row width *width -- and whether the filter runs on the LDS FFT path
+ * backprojector's gather forms stage per angle row for these parameters --
+ * first bin *tlo and row width *width -- and whether the filter runs on the LDS FFT path
  * (*fft_path = 1) or the direct-convolution path (0).  Returns 0 or an error. */
 int raft_fbp_plan_info(const float* angles, const float* paramf, const int* parami, int* tlo, int* width,
                        int* fft_path);
+
+/* Host-only planning query of raft_fbp_device (no device work): the form of
+ * its backprojector for these parameters and rows of this store -- *form = 0:
+ * gather kernels, 1: gather kernels with the angles split over workgroups
+ * (where the workspace fits), 2: matrix cores -- and the bin window that form
+ * stages.  No counterpart in the reference.  Returns 0 or an error. */
+int raft_fbp_form_info(const float* angles, const float* paramf, const int* parami, int store, int* form, int* tlo,
+                       int* width);
 
 /* Host-only planning query of the forward projector (no device work): for
  * the Radon geometry (em = 0: an Ny x Nx image, half extents ax, ay) or the

@@ -594,12 +594,24 @@ static std::vector<double> paired_coefs(const BpGeom& g, size_t pad = BP_MX_TABL
     return v;
 }
 
+// Whether an FBP call runs the matrix backprojector: its rule on sizes, and
+// finite angles.  A NaN or infinite angle has no bins, so the windows of its
+// tiles lie anywhere: the gather forms clamp every window into the rows, the
+// matrix form stages the windows bp_window_matrix has covered, unclamped.
+static bool fbp_matrix(const FbpCfg& c, const float* angles, int store)
+{
+    if (!bp_matrix_form(c.S, c.N, store)) return false;
+    for (int a = 0; a < c.A; ++a)
+        if (!std::isfinite(angles[a])) return false;
+    return true;
+}
+
 // FBP work of one call on stream st; the caller holds D.mu with the device
 // bound.  sync: wait for the stream before returning (the per-call tables in
 // the arena are then free for the next call).
-// mx: run the matrix form of the backprojector (bp_matrix_form of the whole
-// call; it rounds differently from the gather forms, so all blocks of a call
-// take the same one)
+// mx: run the matrix form of the backprojector (fbp_matrix of the whole call;
+// it rounds differently from the gather forms, so all blocks of a call take the
+// same one)
 static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* angles, const FbpCfg& c, int store,
                     hipStream_t st, bool sync, bool mx)
 {
@@ -686,7 +698,7 @@ static void fbp_device(int dev, float* d_obj, const float* d_tomo, const float* 
     bind_device(dev);
     Device& D = device_state(dev);
     std::lock_guard<std::mutex> lk(D.mu);
-    fbp_run(D, d_obj, d_tomo, angles, c, store, st, true, bp_matrix_form(c.S, c.N, store));
+    fbp_run(D, d_obj, d_tomo, angles, c, store, st, true, fbp_matrix(c, angles, store));
 }
 
 // FBP with every intermediate in the library's fixed device scratch array
@@ -769,7 +781,7 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     // the scratch holds fewer than 16 slices its instructions would run mostly
     // empty (2048 x 2048 FP32: 8 slices fit) and the gather form stays.
     const int fit = groups_fit * SB;
-    const bool mx = bp_matrix_form(c.S, N, store) && fit >= 16;
+    const bool mx = fbp_matrix(c, angles, store) && fit >= 16;
     if (mx) {
         const int unit = fit >= 2 * bp_matrix_pack(store) ? 2 * bp_matrix_pack(store) : std::min(bp_matrix_pack(store), fit);
         B = std::min(c.S, std::min(fit, B + unit - 1) / unit * unit);
@@ -2456,6 +2468,24 @@ int raft_fbp_plan_info(const float* angles, const float* paramf, const int* para
         if (tlo) *tlo = g.tlo;
         if (width) *width = g.width;
         if (fft_path) *fft_path = fft_plan(c.npad).ok ? 1 : 0;
+    });
+}
+
+int raft_fbp_form_info(const float* angles, const float* paramf, const int* parami, int store, int* form, int* tlo,
+                       int* width)
+{
+    return guarded([&] {
+        const FbpCfg c = decode_fbp(paramf, parami);
+        if (!angles) fail(RAFT_EINVAL, "null angles");
+        if (store != RAFT_STORE_F32 && store != RAFT_STORE_F16) fail(RAFT_EINVAL, "store must be F32 or F16");
+        const bool mx = fbp_matrix(c, angles, store);
+        BpGeom g;
+        std::vector<float> wa;
+        fbp_geometry(c, angles, g, wa);
+        if (mx) bp_window_matrix(g);
+        if (form) *form = mx ? 2 : (bp_split_workspace(c.S, c.N, c.A, store) ? 1 : 0);
+        if (tlo) *tlo = g.tlo;
+        if (width) *width = g.width;
     });
 }
 

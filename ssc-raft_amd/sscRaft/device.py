@@ -6,7 +6,7 @@ import numpy
 from .rafttypes import CNICE, libraft, raft_check, ctypes
 
 __all__ = ["fbp_device", "lds_read_probe", "radon_device", "eem_device", "eem_kl_device", "batch_device", "lowpass_device",
-           "bst_device", "tem_device", "background_device", "set_profiling", "last_kernel_ms", "fbp_plan_info", "proj_plan_info", "autotune_choices",
+           "bst_device", "tem_device", "background_device", "set_profiling", "last_kernel_ms", "fbp_plan_info", "fbp_form_info", "proj_plan_info", "autotune_choices",
            "autotune_clear", "eem_device_sched",
            "KF_FILTER", "KF_BP", "KF_PROJ", "KF_EMBP"]
 
@@ -264,6 +264,22 @@ def fbp_plan_info(angles, paramf, parami):
     if rc:
         raft_check("raft_fbp_plan_info")
     return tlo.value, width.value, fft.value
+
+
+def fbp_form_info(angles, paramf, parami, store="f32"):
+    """(form, first bin, row width) of the backprojector an fbp_device call
+    with these parameters runs (host only): form 0 = gather kernels, 1 = the
+    same with the angles split over workgroups, 2 = matrix cores."""
+    angles = CNICE(numpy.asarray(angles))
+    paramf = CNICE(numpy.asarray(paramf), numpy.float32)
+    parami = CNICE(numpy.asarray(parami), numpy.int32)
+    form, tlo, width = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    err = libraft.raft_fbp_form_info(angles.ctypes.data_as(ctypes.c_void_p), paramf.ctypes.data_as(ctypes.c_void_p),
+                                     parami.ctypes.data_as(ctypes.c_void_p), 1 if store == "f16" else 0,
+                                     ctypes.byref(form), ctypes.byref(tlo), ctypes.byref(width))
+    if err:
+        raft_check("raft_fbp_form_info")
+    return form.value, tlo.value, width.value
 
 
 def proj_plan_info(angles, Nx, Ny=None, nrays=None, nslices=4, ax=1.0, ay=1.0, em=False):

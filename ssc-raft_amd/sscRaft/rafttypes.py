@@ -85,6 +85,8 @@ libraft.raft_eem_kl_device.argtypes = [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
 libraft.raft_eem_kl_device.restype = _i
 libraft.raft_fbp_plan_info.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp]
 libraft.raft_fbp_plan_info.restype = _i
+libraft.raft_fbp_form_info.argtypes = [_vp, _vp, _vp, _i, _vp, _vp, _vp]
+libraft.raft_fbp_form_info.restype = _i
 libraft.raft_proj_plan_info.argtypes = [_vp, _i, _i, _i, _i, _i, _f, _f, _i, _vp, _vp]
 libraft.raft_proj_plan_info.restype = _i
 libraft.raft_autotune_dump.argtypes = [ctypes.c_char_p, _i]

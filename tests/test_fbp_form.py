@@ -1,0 +1,31 @@
+"""Which backprojector an FBP call takes (raft_fbp_form_info): the matrix form
+only where its staged windows and offsets hold."""
+import numpy as np
+import pytest
+
+GATHER, SPLIT, MATRIX = 0, 1, 2
+
+
+def _angles(a):
+    return (np.linspace(0.0, np.pi, a, endpoint=False) + 0.01).astype(np.float32)
+
+
+def _params(n, a, s, filt=7, pad=2, blocksize=0):
+    paramf = np.array([0.0, 0.0, 0.0, 0.0, 2.0 / n, 2.0 / n, 0.0], np.float32)
+    return paramf, np.array([n, a, s, n, pad, 0, 0, filt, 0, blocksize], np.int32)
+
+
+def _form(ang, n, s, store, **kw):
+    from sscRaft import device as dv
+
+    return dv.fbp_form_info(ang, *_params(n, len(ang), s, **kw), store=store)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("n,a,s,store", [(128, 200, 16, "f16"), (512, 260, 64, "f32")])
+def test_non_finite_angle_keeps_the_gather_form(n, a, s, store, bad):
+    ang = _angles(a)
+    form, tlo, width = _form(ang, n, s, store)
+    assert form == MATRIX and width > n
+    ang[a // 3] = bad
+    assert _form(ang, n, s, store)[0] != MATRIX
