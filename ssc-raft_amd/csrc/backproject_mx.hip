@@ -655,6 +655,17 @@ bool bp_matrix_form(int S, int n, int store)
     return 0.30 * wide + 0.39 * narrow < 0.057e-6 * (double)n * n * S;
 }
 
+// One launch addresses an angle's rows with 32-bit byte offsets, and takes no
+// more slice groups than the gather form does (a larger call is left to that
+// form, which refuses it).  A row holds less than 1.5 n + 128 bins.
+constexpr long long BM_GROUPS = 65535, BM_BYTES = (1LL << 32) - 8192;
+bool bp_matrix_fits(int slices, int n, int store)
+{
+    const int pack = bp_matrix_pack(store), sb = store == RAFT_STORE_F16 ? BP_SLICES_F16 : BP_SLICES_F32;
+    const long long groups = ((long long)slices + pack - 1) / pack * (pack / sb);
+    return groups <= BM_GROUPS && groups * (3LL * n / 2 + 128) * (long long)bp_matrix_entry(store) <= BM_BYTES;
+}
+
 int bp_matrix_pack(int store) { return store == RAFT_STORE_F16 ? 32 : 16; }
 
 size_t bp_matrix_entry(int store) { return store == RAFT_STORE_F16 ? 16 : 24; }
@@ -708,6 +719,8 @@ void launch_backproject_mx(const BpArgs& b, int store, hipStream_t st)
     const size_t need = (size_t)a.G * a.A * a.W * (checked ? 16 : bp_matrix_entry(store));
     if (b.q_bytes && need > b.q_bytes)
         fail(RAFT_EINVAL, "internal: backprojection would read past its staged rows");
+    if (a.G > BM_GROUPS || (!checked && (long long)a.G * a.W * (long long)bp_matrix_entry(store) > BM_BYTES))
+        fail(RAFT_EUNSUPPORTED, "too many slice groups for one backprojection launch");
     const BmPlan p = bm_plan(b.S, b.n, f16);
     if (checked) bm_launch_plan<true>(a, p, f16, st);
     else bm_launch_plan<false>(a, p, f16, st);

@@ -29,3 +29,17 @@ def test_non_finite_angle_keeps_the_gather_form(n, a, s, store, bad):
     assert form == MATRIX and width > n
     ang[a // 3] = bad
     assert _form(ang, n, s, store)[0] != MATRIX
+
+
+@pytest.mark.parametrize("n,s,store", [
+    (64, 6_400_000, "f32"),   # 4.5 GB of rows an angle: 32-bit offsets would wrap
+    (8, 36_000_000, "f16"),
+    (8, 524_281, "f16"),      # one slice past 65535 groups, which the gather form refuses
+    (64, 262_141, "f32"),
+])
+def test_blocks_past_one_launch_keep_the_gather_form(n, s, store):
+    ang = _angles(400)
+    assert _form(ang, n, s, store)[0] != MATRIX
+    # in blocks each launch is small
+    form, _, width = _form(ang, n, s, store, blocksize=4096)
+    assert form == MATRIX and width <= 1.5 * n + 128
