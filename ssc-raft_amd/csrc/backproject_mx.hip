@@ -629,8 +629,8 @@ static BmPlan bm_plan(int S, int n, bool f16)
     return p;
 }
 
-// Whether an FBP call of S slices of n x n runs here.  Backprojection
-// time, gather form -> this file, n angles and rays (ms):
+// Whether an FBP call of S slices of n x n from A angles runs here.
+// Backprojection time, gather form -> this file, n angles and rays (ms):
 //   FP32 rows   S = 16            32             64
 //     n =  512  0.188 -> 0.206  0.277 -> 0.298  0.531 -> 0.465
 //     n = 1024  0.985 -> 1.040  1.97  -> 1.54   3.96  -> 2.91
@@ -644,15 +644,34 @@ static BmPlan bm_plan(int S, int n, bool f16)
 // workgroup on each of 256 CUs) takes 0.30 us and a round of narrow ones (two on
 // each) 0.39 us, the gather form 0.057 us per 10^6 pixels and slices (a little
 // more where it cannot fill the chip).
-bool bp_matrix_form(int S, int n, int store)
+// The image leaves through LDS here, 0.8 to 0.9 us per 10^6 pixels and slices more
+// than in the gather form, which the angles have to earn back.  Few angles (us):
+//   FP32 2048, S = 64   A = 2  190 -> 447   32  559 -> 670   64  1010 -> 930
+//         512, S = 200       35 -> 77          113 -> 138        201 -> 205
+//         200, S = 150       12 -> 14           31 -> 22          52 -> 30
+//   FP16 2048, S = 32       120 -> 220        215 -> 219        394 -> 277
+//        1024, S = 16        16 -> 34          37 -> 50          65 -> 70
+//          64, S = 70         7 -> 16          18 -> 22          31 -> 29
+// There the gather form takes 0.44 ns a workgroup and angle and 0.14 us an angle
+// (FP16 0.6 ns and 0.2 us, 0.37 us at least), a round here 0.27 us (narrow 0.36, FP16
+// 0.22; FP16's small images 2.6 us and 0.09 us a slice of a pack besides).
+bool bp_matrix_form(int S, int n, int A, int store)
 {
     if (S < 16 || n < 1) return false;
-    if (store == RAFT_STORE_F16) return true;
-    const BmPlan p = bm_plan(S, n, false);
+    const bool f16 = store == RAFT_STORE_F16;
+    const BmPlan p = bm_plan(S, n, f16);
     const long long tiles = bm_tiles(n);
     const double wide = (double)((tiles * p.wide + BM_CUS - 1) / BM_CUS);
     const double narrow = (double)((tiles * p.narrow + 2 * BM_CUS - 1) / (2 * BM_CUS));
-    return 0.30 * wide + 0.39 * narrow < 0.057e-6 * (double)n * n * S;
+    const double image = 1.0e-6 * (double)n * n * S;
+    const int sb = f16 ? BP_SLICES_F16 : BP_SLICES_F32;
+    const double groups = (double)bp_tiles(n) * ((S + sb - 1) / sb); // workgroups of the gather form
+    if (f16) {
+        const double once = 2.6 + 0.09 * std::min(S, Form<2>::SLICES) + 0.8 * image;
+        return A * 0.22 * (wide + narrow) + once < A * std::max(0.37, 0.6e-3 * groups + 0.2);
+    }
+    return 0.30 * wide + 0.39 * narrow < 0.057 * image &&
+           A * (0.27 * wide + 0.36 * narrow) + 0.9 * image < A * (0.437e-3 * groups + 0.14);
 }
 
 // One launch addresses an angle's rows with 32-bit byte offsets, and takes no

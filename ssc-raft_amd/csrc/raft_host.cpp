@@ -600,7 +600,7 @@ static std::vector<double> paired_coefs(const BpGeom& g, size_t pad = BP_MX_TABL
 // matrix form stages the windows bp_window_matrix has covered, unclamped.
 static bool fbp_matrix(const FbpCfg& c, const float* angles, int store)
 {
-    if (!bp_matrix_form(c.S, c.N, store)) return false;
+    if (!bp_matrix_form(c.S, c.N, c.A, store)) return false;
     if (!bp_matrix_fits(c.blocksize > 0 ? std::min(c.blocksize, c.S) : c.S, c.N, store)) return false;
     for (int a = 0; a < c.A; ++a)
         if (!std::isfinite(angles[a])) return false;

@@ -229,9 +229,9 @@ struct BpArgs {
 void launch_backproject(const BpArgs& a, int store, hipStream_t st);
 // bytes of its workspace where few tiles should be split over the angles, else 0
 size_t bp_split_workspace(int S, int n, int A, int store);
-// whether an FBP call of S slices of n x n runs the matrix form (chunk =
-// BP_MX); decided once per call, so blocks of a call agree
-bool bp_matrix_form(int S, int n, int store);
+// whether an FBP call of S slices of n x n from A angles runs the matrix form
+// (chunk = BP_MX); decided once per call, so blocks of a call agree
+bool bp_matrix_form(int S, int n, int A, int store);
 // whether a block of this many slices is within one launch's addressing
 bool bp_matrix_fits(int slices, int n, int store);
 // slices of its smallest pack: blocks of a call are multiples of it

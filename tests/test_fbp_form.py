@@ -43,3 +43,25 @@ def test_blocks_past_one_launch_keep_the_gather_form(n, s, store):
     # in blocks each launch is small
     form, _, width = _form(ang, n, s, store, blocksize=4096)
     assert form == MATRIX and width <= 1.5 * n + 128
+
+
+@pytest.mark.parametrize("n,s,store,few,many", [
+    # angles at which the matrix form took longer, and at which it gains
+    (2048, 64, "f32", 32, 128),
+    (2048, 32, "f32", 24, 128),
+    (2048, 16, "f32", 96, 2048),
+    (1024, 64, "f32", 16, 96),
+    (512, 200, "f32", 48, 512),
+    (512, 64, "f32", 32, 256),
+    (200, 150, "f32", 8, 48),
+    (2048, 32, "f16", 16, 64),
+    (1024, 16, "f16", 64, 512),
+    (512, 64, "f16", 24, 96),
+    (200, 70, "f16", 32, 200),
+    (64, 70, "f16", 32, 96),
+    (16, 16, "f16", 24, 48),
+])
+def test_few_angles_keep_the_gather_form(n, s, store, few, many):
+    assert _form(_angles(few), n, s, store)[0] != MATRIX
+    assert _form(_angles(2), n, s, store)[0] != MATRIX
+    assert _form(_angles(many), n, s, store)[0] == MATRIX
