@@ -624,7 +624,8 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
 
     FilterTables& F = filter_tables(D, c, st);
     TableSet tb(D);
-    const TabRef dcA = tb.add(g.cA), dcB = tb.add(g.cB), dwa = tb.add(wa), dcs = tb.add(paired_coefs(g));
+    const TabRef dcA = tb.add(g.cA), dcB = tb.add(g.cB), dwa = tb.add(wa);
+    const TabRef dcs = tb.add(mx ? paired_coefs(g) : std::vector<double>());
     tb.upload(st);
     if (!sync) tb.keep_alive();
 
@@ -665,7 +666,7 @@ static void fbp_run(Device& D, float* d_obj, const float* d_tomo, const float* a
         ba.xc = g.xc; ba.c0 = g.c0;
         ba.n = N; ba.A = A; ba.S = nb; ba.tlo = g.tlo; ba.W = g.width; ba.mode = 0;
         ba.q_bytes = (size_t)((B + SB - 1) / SB) * per_group;
-        ba.cs = dcs.as<double>();
+        ba.cs = mx ? dcs.as<double>() : nullptr;
         // angle chunk: tuned on this block's rows (the timed launches write
         // the same output as the final one)
         ba.chunk = mx ? BP_MX
