@@ -578,14 +578,19 @@ static BpKArgs bp_kargs(const BpArgs& b)
 // workgroup on half of the CUs.  1 slice of 512 x 512, 512 angles: 159 us whole,
 // 59 split (about 2048 workgroups; 62 at 768); 4 slices 159 and 80 (134 MB of
 // partial sums); 256 x 256, 256 angles 84 and 16; 64 x 64, 64 angles 24 and 12.
-// Above 256 tiles every CU has work (1024 x 1024: 512 tiles).
+// Above 256 tiles every CU has work (1024 x 1024: 512 tiles).  The more of the CUs
+// the whole form fills, the more angles the partial sums need to pay: with 64 angles
+// 128 workgroups 25.2 -> 23.2 us, 182 26.0 -> 25.4 (and the filter 3 us slower, its
+// tables gone from L2), 256 25.8 -> 33.6; 256 with 128 angles 45.5 -> 46.8, 160 55.4 ->
+// 55.0, 200 67.5 -> 63.7.
 constexpr size_t BP_SPLIT_CAP = (size_t)192 << 20;
 
 size_t bp_split_workspace(int S, int n, int A, int store)
 {
     const long long wgs = (long long)bp_tiles(n) * ((S + 3) / 4);
     const size_t bytes = (size_t)((A + BP_GROUP - 1) / BP_GROUP) * S * n * n * sizeof(float);
-    if (store != RAFT_STORE_F32 || wgs > 256 || A < 4 * BP_GROUP || bytes > BP_SPLIT_CAP) return 0;
+    const long long least = 4 * BP_GROUP + std::max(0LL, wgs - 128) * 5 / 8; // 64 angles, 144 at 256 workgroups
+    if (store != RAFT_STORE_F32 || wgs > 256 || A < least || bytes > BP_SPLIT_CAP) return 0;
     return bytes;
 }
 

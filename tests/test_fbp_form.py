@@ -65,3 +65,15 @@ def test_few_angles_keep_the_gather_form(n, s, store, few, many):
     assert _form(_angles(few), n, s, store)[0] != MATRIX
     assert _form(_angles(2), n, s, store)[0] != MATRIX
     assert _form(_angles(many), n, s, store)[0] == MATRIX
+
+
+@pytest.mark.parametrize("n,s,whole,split", [
+    (512, 1, 63, 64),     # 128 workgroups
+    (400, 8, 64, 128),    # 182
+    (512, 8, 128, 160),   # 256
+    (600, 4, 64, 128),    # 190
+    (64, 9, 63, 64),
+])
+def test_few_angles_are_not_split(n, s, whole, split):
+    assert _form(_angles(whole), n, s, "f32")[0] == GATHER
+    assert _form(_angles(split), n, s, "f32")[0] == SPLIT
