@@ -96,18 +96,15 @@ int raft_fbp_device(int device, float* d_obj, const float* d_tomo, const float* 
 /* raft_fbp_device that allocates no device memory.  No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * arguments, same kernels and the same output bit for bit, but for two cases
- * that differ by rounding: where the array holds fewer than 16 slices, a call
- * that raft_fbp_device sums on the matrix cores keeps the gather kernels here;
- * where one slice group fits only without the faster filter forms' tables, the
- * general ones run.  The filter and
- * angle tables and the filtered rows live in one fixed device array of
- * RAFT_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
- * process ends, and the slices run in blocks of as many slice groups (4 slices
- * for F32 rows, 8 for F16) as fit there.  A geometry whose tables plus one
- * slice group of rows (nangles x staged width x 16 bytes) exceed the array is
- * refused with RAFT_EUNSUPPORTED (2048 angles x 2048 rays at pad 2 needs
- * 90.75 MiB per group).  Synchronous: it waits for its stream before returning.
+ * arguments, same kernels and the same output bit for bit.  The filter and
+ * angle tables and the filtered rows live in one fixed device array that a GPU
+ * holds from the first such call on it until the process ends (4 x
+ * RAFT_NOALLOC_SCRATCH_BYTES + 4 MiB, so that the matrix backprojector's 16
+ * slices fit wherever one slice group does), and the slices run in blocks of as
+ * many slice groups (4 slices for F32 rows, 8 for F16) as fit there.  A geometry
+ * whose filter and angle tables plus one slice group of rows (nangles x staged
+ * width x 16 bytes) exceed RAFT_NOALLOC_SCRATCH_BYTES is refused with
+ * RAFT_EUNSUPPORTED (2048 angles x 2048 rays at pad 2 needs 90.75 MiB per group).  Synchronous: it waits for its stream before returning.
  * Calls on one device share its array and are serialised by the library. */
 #define RAFT_NOALLOC_SCRATCH_BYTES (256ull << 20)
 int raft_fbp_device_noalloc(int device, float* d_obj, const float* d_tomo, const float* angles,

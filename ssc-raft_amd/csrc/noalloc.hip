@@ -1,8 +1,9 @@
 // noalloc.hip -- the fixed device scratch array of raft_fbp_device_noalloc.
 //
 // `scratch` is a file-scope __device__ array: every GPU the library runs on
-// holds its own copy, at its own address, from the moment the library's code
-// is loaded there until the process ends.  In host code the array's name is a
+// holds its own copy, at its own address, from the moment this file's code is
+// loaded there (at the first noalloc_scratch(), which takes 0.4 ms a MiB: 0.1 s
+// for 256 MiB, 0.4 s for the 1028) until the process ends.  In host code the array's name is a
 // host-side stand-in and not a device address, so host code never hands it to
 // a kernel or a copy.  noalloc_scratch() asks the runtime for the device
 // address once per device, with that device current, checks the result and
@@ -18,7 +19,7 @@
 
 #include "raft_internal.hpp"
 
-static __device__ __align__(256) unsigned char scratch[RAFT_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[raft::NOALLOC_ARRAY_BYTES];
 
 namespace raft {
 

@@ -708,8 +708,8 @@ static void fbp_device(int dev, float* d_obj, const float* d_tomo, const float* 
 // cosines, sines and weights, then as many slice groups of filtered rows as
 // fit.  The volume runs in blocks of that many groups through the same
 // kernels with the same arguments as fbp_run, so the output is fbp_run's bit
-// for bit (slice groups are independent, and every angle chunk of the
-// backprojector gives the same sums).  Nothing here allocates device memory:
+// for bit (slice groups are independent, and every angle chunk and every pack
+// of the backprojector gives the same sums).  Nothing here allocates device memory:
 // no workspace, no table arena, no cached device filter tables, no tuning
 // runs (the backprojector takes the tuner's cached chunk or its default).
 // Nothing in the scratch must start at zero: the filter writes every entry of
@@ -752,44 +752,42 @@ static void fbp_device_noalloc(int dev, float* d_obj, const float* d_tomo, const
     const size_t oH = put(F->H.data(), F->H.size() * sizeof(float2));
     const size_t oTw = put(F->tw.data(), F->tw.size() * sizeof(float2));
     const size_t oG = put(F->g.data(), F->g.size() * sizeof(double));
-    // the tables of the faster filter forms, where a slice group of rows still
-    // fits behind them (else the general forms: the same sums, rounded apart)
-    const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
-    const size_t per_group = (size_t)A * g.width * 16;
-    const size_t cap = (size_t)RAFT_NOALLOC_SCRATCH_BYTES;
-    const size_t conv_bytes = (F->spec.size() + F->ctw.size() + F->edge.size()) * sizeof(double) + 3 * 256;
-    const bool conv = F->conv.len > 0 && host.size() + conv_bytes + (size_t)A * 20 + 4 * 256 + per_group <= cap;
-    const bool dif = !F->difH.empty() &&
-                     host.size() + (F->difH.size() + F->diftw.size()) * sizeof(float2) + (size_t)A * 20 + 7 * 256 + per_group <= cap;
-    const size_t oDifH = dif ? put(F->difH.data(), F->difH.size() * sizeof(float2)) : 0;
-    const size_t oDifTw = dif ? put(F->diftw.data(), F->diftw.size() * sizeof(float2)) : 0;
-    const size_t oSpec = conv ? put(F->spec.data(), F->spec.size() * sizeof(double)) : 0;
-    const size_t oCtw = conv ? put(F->ctw.data(), F->ctw.size() * sizeof(double)) : 0;
-    const size_t oEdge = conv ? put(F->edge.data(), F->edge.size() * sizeof(double)) : 0;
     const size_t oA = put(g.cA.data(), (size_t)A * sizeof(double));
     const size_t oB = put(g.cB.data(), (size_t)A * sizeof(double));
     const size_t oW = put(wa.data(), (size_t)A * sizeof(float));
-    const size_t oRows = (host.size() + 255) & ~(size_t)255;
-
-    if (oRows > cap || cap - oRows < per_group)
-        fail(RAFT_EUNSUPPORTED, "raft_fbp_device_noalloc: tables (" + std::to_string(oRows) +
+    const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
+    const size_t per_group = (size_t)A * g.width * 16;
+    const size_t cap = (size_t)RAFT_NOALLOC_SCRATCH_BYTES, tables = (host.size() + 255) & ~(size_t)255;
+    if (tables > cap || cap - tables < per_group)
+        fail(RAFT_EUNSUPPORTED, "raft_fbp_device_noalloc: tables (" + std::to_string(tables) +
                                     " bytes) and one slice group of filtered rows (" + std::to_string(per_group) +
-                                    " bytes) exceed the fixed scratch of " + std::to_string(cap) + " bytes");
-    const int groups_fit = (int)std::min<size_t>((cap - oRows) / per_group, 1 << 20);
+                                    " bytes) exceed the fixed scratch's " + std::to_string(cap) + " bytes for them");
+    // the tables of the filter forms that have some, and the matrix form's pairs in
+    // place of the two tables
+    const bool mx = fbp_matrix(c, angles, store);
+    const bool dif = !F->difH.empty(), conv = F->conv.len > 0;
+    const size_t oDifH = put(F->difH.data(), F->difH.size() * sizeof(float2));
+    const size_t oDifTw = put(F->diftw.data(), F->diftw.size() * sizeof(float2));
+    const size_t oSpec = put(F->spec.data(), F->spec.size() * sizeof(double));
+    const size_t oCtw = put(F->ctw.data(), F->ctw.size() * sizeof(double));
+    const size_t oEdge = put(F->edge.data(), F->edge.size() * sizeof(double));
+    if (mx) {
+        const std::vector<double> cs = paired_coefs(g, 0);
+        std::memcpy(host.data() + oA, cs.data(), cs.size() * sizeof(double));
+    }
+    const size_t oRows = (host.size() + 255) & ~(size_t)255;
+    if (oRows + 4 * per_group > NOALLOC_ARRAY_BYTES) fail(RAFT_EINVAL, "internal: the scratch array is too small");
+
+    const int groups_fit = (int)std::min<size_t>((NOALLOC_ARRAY_BYTES - oRows) / per_group, 1 << 20);
     int B = c.blocksize > 0 ? std::min(c.blocksize, c.S) : c.S;
     B = std::min(c.S, ((B + SB - 1) / SB) * SB);
     B = std::min(B, groups_fit * SB);
-    // The matrix form where fbp_run takes it, in blocks of whole packs.  Where
-    // the scratch holds fewer than 16 slices its instructions would run mostly
-    // empty (2048 x 2048 FP32: 8 slices fit) and the gather form stays.
-    const int fit = groups_fit * SB;
-    const bool mx = fbp_matrix(c, angles, store) && fit >= 16;
+    // the matrix form runs in blocks of whole packs: four slice groups always fit,
+    // which is a pack of either store
     if (mx) {
-        const int unit = fit >= 2 * bp_matrix_pack(store) ? 2 * bp_matrix_pack(store) : std::min(bp_matrix_pack(store), fit);
+        const int fit = groups_fit * SB;
+        const int unit = bp_matrix_pack(store) * (fit >= 2 * bp_matrix_pack(store) ? 2 : 1);
         B = std::min(c.S, std::min(fit, B + unit - 1) / unit * unit);
-        // its coefficient pairs take the place of the two tables
-        const std::vector<double> cs = paired_coefs(g, 0);
-        std::memcpy(host.data() + oA, cs.data(), cs.size() * sizeof(double));
     }
 
     bind_device(dev);

@@ -345,8 +345,14 @@ void launch_background(float* data, const float* flat, const float* dark, int R,
 // p[0 .. n) = v (a kernel, so it may be captured into a graph)
 void launch_fill(float* p, long long n, float v, hipStream_t st);
 
+// The scratch array of raft_fbp_device_noalloc: four times what one slice group
+// and its tables may take, so that a pack of the matrix form (4 groups) fits
+// wherever a group does, and the tables of the faster filter forms.  With room for
+// fewer than 16 slices (256 MiB: 8 of 2048 x 2048 in FP32) its packs would run mostly
+// empty, and the gather form would round differently from raft_fbp_device.
+constexpr size_t NOALLOC_ARRAY_BYTES = 4 * (size_t)RAFT_NOALLOC_SCRATCH_BYTES + ((size_t)4 << 20);
 // device address of this device's copy of the fixed scratch array of
-// RAFT_NOALLOC_SCRATCH_BYTES (noalloc.hip); dev must be the current device
+// NOALLOC_ARRAY_BYTES (noalloc.hip); dev must be the current device
 void* noalloc_scratch(int dev);
 
 // autotuner (autotune.cpp): the cached choice for key, else the fastest of
