@@ -571,7 +571,7 @@ constexpr int CV_MAX_CHUNKS = 16;
 constexpr int CV_MIN_N = 128;
 typedef double d2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ int cpix(int e) { return e + (e >> 3); }
-size_t conv_lds(int len) { return sizeof(double) * 2 * ((size_t)len + (size_t)(len >> 3) + 1); }
+__host__ __device__ constexpr size_t conv_lds(int len) { return sizeof(double) * 2 * ((size_t)len + (size_t)(len >> 3) + 1); }
 
 struct ConvK {
     const d2* spec;     // [chunks][len], permuted as the forward passes leave it, 1 / len folded in
@@ -795,7 +795,16 @@ template <typename OT> __global__ __launch_bounds__(CV_THREADS, 4) void k_filter
     case 5: bad = conv_first<5>(a, ix, c, z); break;
     default: bad = conv_first<8>(a, ix, c, z); break;
     }
-    if (__syncthreads_or(bad)) {
+    // over the workgroup, through LDS of its own behind the transform (a static array,
+    // as __syncthreads_or has, would not fit beside the longest rows the direct sum takes)
+    int* any = reinterpret_cast<int*>(conv_smem + conv_lds(c.len));
+    bad = __any(bad);
+    if ((threadIdx.x & 63) == 0) any[threadIdx.x >> 6] = bad;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < CV_THREADS / 64; ++w) bad |= any[w] != 0;
+    if (bad) {
+        __syncthreads(); // `any` is read
         // a row that is not finite must not reach the other of the pair
         load_pair<CV_THREADS>(a, ix, reinterpret_cast<float2*>(z));
         __syncthreads();
@@ -856,7 +865,7 @@ template <typename OT> void launch_conv(const FilterK& k, const FilterArgs& a, h
     c.rows = (unsigned)((long long)((k.S + k.SB - 1) / k.SB) * k.A);
     const long long blocks = ((long long)c.rows + 7) / 8 * 8 * (k.SB / 2) * c.count;
     if (blocks > 0x7fffffffLL) fail(RAFT_EUNSUPPORTED, "too many sinogram rows for one filter launch");
-    const size_t lds = std::max(conv_lds(p.len), sizeof(float2) * lds_elems(k.npad));
+    const size_t lds = std::max(conv_lds(p.len) + CV_THREADS / 64 * sizeof(int), sizeof(float2) * lds_elems(k.npad));
     RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_filter_conv<OT>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_filter_conv<OT>), dim3((unsigned)blocks), dim3(CV_THREADS), lds, st, k, c);
