@@ -569,6 +569,9 @@ constexpr int CV_MAX_CHUNKS = 16;
 // padded rows from here on: n = 98 takes 10.2 us direct and 13.6 by transforms
 // (320 row pairs), n = 202 43.7 and 22.8 (1440 pairs)
 constexpr int CV_MIN_N = 128;
+// binary orders of magnitude between two rows from which each is summed by itself:
+// below, the larger one's rounding stays 2^8 below an FP32 rounding of the smaller
+constexpr unsigned CV_APART = 20;
 typedef double d2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ int cpix(int e) { return e + (e >> 3); }
 __host__ __device__ constexpr size_t conv_lds(int len) { return sizeof(double) * 2 * ((size_t)len + (size_t)(len >> 3) + 1); }
@@ -692,22 +695,38 @@ template <int R, bool INV, typename V> __device__ __forceinline__ void ztwiddle(
     for (int q = 1; q < R; ++q) v[q] = zmul(v[q], INV ? zconj(w[q]) : w[q]);
 }
 
-// the first forward pass, from the rows; returns whether a sample read is not finite
+// maximum over the wave, in lane 63
+__device__ __forceinline__ unsigned wave_max(unsigned v)
+{
+#define RAFT_DPP_MAX(CTRL) v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false))
+    RAFT_DPP_MAX(0x111); // row_shr 1, 2, 4, 8: lane 15 of every row of 16
+    RAFT_DPP_MAX(0x112);
+    RAFT_DPP_MAX(0x114);
+    RAFT_DPP_MAX(0x118);
+    RAFT_DPP_MAX(0x142); // row_bcast 15, 31
+    RAFT_DPP_MAX(0x143);
+#undef RAFT_DPP_MAX
+    return v;
+}
+
+// the first forward pass, from the rows; returns the bits of the largest magnitude read
+// of each row (a NaN's lie above an infinity's)
 template <int R>
-__device__ __forceinline__ bool conv_first(const FilterK& a, const PairIdx& ix, const ConvK& c, d2* z)
+__device__ __forceinline__ uint2 conv_first(const FilterK& a, const PairIdx& ix, const ConvK& c, d2* z)
 {
     const bool h0 = ix.s0 < a.S, h1 = ix.s0 + 1 < a.S;
     const float* r0 = a.tomo + ((size_t)ix.s0 * a.A + ix.a) * a.N;
     const float* r1 = r0 + (size_t)a.A * a.N;
     const int M = c.len / R;
-    bool bad = false;
+    uint2 m = make_uint2(0u, 0u);
     for (int j = threadIdx.x; j < M; j += CV_THREADS) {
         d2 v[R];
 #pragma unroll
         for (int t = 0; t < R; ++t) {
             const int i = j + t * M;
             const float x0 = h0 && i < a.N ? r0[i] : 0.0f, x1 = h1 && i < a.N ? r1[i] : 0.0f;
-            bad |= !((x0 - x0) + (x1 - x1) == 0.0f);
+            m.x = max(m.x, __float_as_uint(x0) & 0x7fffffffu);
+            m.y = max(m.y, __float_as_uint(x1) & 0x7fffffffu);
             v[t] = d2{(double)x0, (double)x1};
         }
         zdft<R, false>(v);
@@ -715,7 +734,7 @@ __device__ __forceinline__ bool conv_first(const FilterK& a, const PairIdx& ix, 
 #pragma unroll
         for (int t = 0; t < R; ++t) z[cpix(j + t * M)] = v[t];
     }
-    return bad;
+    return m;
 }
 // a pass over blocks of B elements
 template <int R, bool INV> __device__ __forceinline__ void conv_pass(const ConvK& c, int B, d2* z)
@@ -735,7 +754,8 @@ template <int R, bool INV> __device__ __forceinline__ void conv_pass(const ConvK
 }
 // the last inverse pass, to the bins
 template <typename OT, int R>
-__device__ __forceinline__ void conv_last(const FilterK& a, const PairIdx& ix, const ConvK& c, int T0, const d2* z)
+__device__ __forceinline__ void conv_last(const FilterK& a, const PairIdx& ix, const ConvK& c, int T0, uint2 m,
+                                          const d2* z)
 {
     const float* r0 = a.tomo + ((size_t)ix.s0 * a.A + ix.a) * a.N;
     const float* r1 = r0 + (size_t)a.A * a.N;
@@ -755,7 +775,8 @@ __device__ __forceinline__ void conv_last(const FilterK& a, const PairIdx& ix, c
             const int T = T0 + j + t * M;
             if (T < lo || T >= hi) continue;
             const double e0 = c.edge[T], e1 = c.edge[a.npad + T];
-            store_sum<OT>(a, ix, T - a.tlo, fma(u0, e1, fma(l0, e0, v[t].x)), fma(u1, e1, fma(l1, e0, v[t].y)));
+            store_sum<OT>(a, ix, T - a.tlo, m.x ? fma(u0, e1, fma(l0, e0, v[t].x)) : 0.0,
+                          m.y ? fma(u1, e1, fma(l1, e0, v[t].y)) : 0.0);
         }
     }
 }
@@ -788,24 +809,32 @@ template <typename OT> __global__ __launch_bounds__(CV_THREADS, 4) void k_filter
         return;
     }
 
-    bool bad;
+    uint2 m;
     switch (c.radix[0]) {
-    case 3: bad = conv_first<3>(a, ix, c, z); break;
-    case 4: bad = conv_first<4>(a, ix, c, z); break;
-    case 5: bad = conv_first<5>(a, ix, c, z); break;
-    default: bad = conv_first<8>(a, ix, c, z); break;
+    case 3: m = conv_first<3>(a, ix, c, z); break;
+    case 4: m = conv_first<4>(a, ix, c, z); break;
+    case 5: m = conv_first<5>(a, ix, c, z); break;
+    default: m = conv_first<8>(a, ix, c, z); break;
     }
-    // over the workgroup, through LDS of its own behind the transform (a static array,
-    // as __syncthreads_or has, would not fit beside the longest rows the direct sum takes)
-    int* any = reinterpret_cast<int*>(conv_smem + conv_lds(c.len));
-    bad = __any(bad);
-    if ((threadIdx.x & 63) == 0) any[threadIdx.x >> 6] = bad;
+    // over the workgroup, through LDS of its own behind the transform (a static array
+    // would not fit beside the longest rows the direct sum takes)
+    uint2* part = reinterpret_cast<uint2*>(conv_smem + conv_lds(c.len));
+    m.x = wave_max(m.x);
+    m.y = wave_max(m.y);
+    if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = m;
     __syncthreads();
+    m = make_uint2(0u, 0u);
 #pragma unroll
-    for (int w = 0; w < CV_THREADS / 64; ++w) bad |= any[w] != 0;
-    if (bad) {
-        __syncthreads(); // `any` is read
-        // a row that is not finite must not reach the other of the pair
+    for (int w = 0; w < CV_THREADS / 64; ++w) {
+        m.x = max(m.x, part[w].x);
+        m.y = max(m.y, part[w].y);
+    }
+    // The rows share the transform's rounding, 2^-52 of the larger one: a pair too far
+    // apart takes the direct sum, and a row of zeros stays zero.
+    const bool apart = m.x > 0u && m.y > 0u && max(m.x, m.y) - min(m.x, m.y) >= CV_APART << 23;
+    if (max(m.x, m.y) >= 0x7f800000u || apart) {
+        __syncthreads(); // `part` is read
+        // a row that is not finite, or far larger, must not reach the other of the pair
         load_pair<CV_THREADS>(a, ix, reinterpret_cast<float2*>(z));
         __syncthreads();
         direct_window<OT, CV_THREADS>(a, ix, reinterpret_cast<const float2*>(z), max(T0 - a.tlo, 0),
@@ -842,10 +871,10 @@ template <typename OT> __global__ __launch_bounds__(CV_THREADS, 4) void k_filter
         __syncthreads();
     }
     switch (c.radix[0]) {
-    case 3: conv_last<OT, 3>(a, ix, c, T0, z); break;
-    case 4: conv_last<OT, 4>(a, ix, c, T0, z); break;
-    case 5: conv_last<OT, 5>(a, ix, c, T0, z); break;
-    default: conv_last<OT, 8>(a, ix, c, T0, z); break;
+    case 3: conv_last<OT, 3>(a, ix, c, T0, m, z); break;
+    case 4: conv_last<OT, 4>(a, ix, c, T0, m, z); break;
+    case 5: conv_last<OT, 5>(a, ix, c, T0, m, z); break;
+    default: conv_last<OT, 8>(a, ix, c, T0, m, z); break;
     }
 }
 
@@ -865,7 +894,7 @@ template <typename OT> void launch_conv(const FilterK& k, const FilterArgs& a, h
     c.rows = (unsigned)((long long)((k.S + k.SB - 1) / k.SB) * k.A);
     const long long blocks = ((long long)c.rows + 7) / 8 * 8 * (k.SB / 2) * c.count;
     if (blocks > 0x7fffffffLL) fail(RAFT_EUNSUPPORTED, "too many sinogram rows for one filter launch");
-    const size_t lds = std::max(conv_lds(p.len) + CV_THREADS / 64 * sizeof(int), sizeof(float2) * lds_elems(k.npad));
+    const size_t lds = std::max(conv_lds(p.len) + CV_THREADS / 64 * sizeof(uint2), sizeof(float2) * lds_elems(k.npad));
     RAFT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_filter_conv<OT>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_filter_conv<OT>), dim3((unsigned)blocks), dim3(CV_THREADS), lds, st, k, c);
