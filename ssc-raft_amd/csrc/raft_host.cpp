@@ -976,16 +976,21 @@ static void lowpass_device(int dev, float* d_tomo, const float* paramf, const in
 // in turns leave CUs idle at each end: 16 slices of 1024 x 1024, 180 angles take
 // 0.75 / 0.64 / 0.56 / 0.53 ms with 64 / 128 / 256 / 512 MB)
 constexpr size_t PROJ_TILE_CAP = (size_t)512 << 20;
-static void proj_tiles(Device& D, ProjArgs& p, const std::vector<double>& c, const std::vector<double>& s, int prc, int S,
-                       size_t budget)
+// its plan (ProjArgs::tile_rs) for a staged plan prc; 0: it does not run.  It reads one
+// orientation of the image, so the callers leave the transposed one out.
+static int proj_tile_form(const RayGeom& g, const std::vector<double>& c, const std::vector<double>& s, int prc,
+                          size_t budget)
 {
-    if (prc > 0) return;
-    const int rs = proj_tile_plan(p.g, c.data(), s.data());
-    const size_t bytes = proj_tile_workspace(p.g, rs, S, std::min(PROJ_TILE_CAP, budget / 8));
-    if (!bytes) return;
+    if (prc > 0) return 0;
+    const int rs = proj_tile_plan(g, c.data(), s.data());
+    return proj_tile_workspace(g, rs, 4, std::min(PROJ_TILE_CAP, budget / 8)) ? rs : 0;
+}
+static void proj_tiles(Device& D, ProjArgs& p, int rs, int S, size_t budget)
+{
+    if (!rs) return;
     p.tile_rs = rs;
-    p.tile_part = D.workspace<14>(bytes);
-    p.tile_bytes = bytes;
+    p.tile_bytes = proj_tile_workspace(p.g, rs, S, std::min(PROJ_TILE_CAP, budget / 8));
+    p.tile_part = D.workspace<14>(p.tile_bytes);
 }
 
 static void radon_device(int dev, float* d_proj, const float* d_obj, const float* angles, int Nx, int Ny, int nrays,
@@ -1014,10 +1019,13 @@ static void radon_device(int dev, float* d_proj, const float* d_obj, const float
     const size_t img = (size_t)Nx * Ny;
     int B = ((nslices + 3) / 4) * 4;
     const size_t budget = block_budget();
-    while (B > 4 && (size_t)B * img * 8 > budget) B = (((B + 1) / 2 + 3) / 4) * 4;
+    int prc = proj_plan(g, cv.data(), sv.data(), B, true);
+    const int rs = proj_tile_form(g, cv, sv, prc, budget);
+    const int whole = B;
+    while (B > 4 && (size_t)B * img * (rs ? 4 : 8) > budget) B = (((B + 1) / 2 + 3) / 4) * 4;
+    if (prc > 0 && B < whole) prc = proj_plan(g, cv.data(), sv.data(), B, true);
     float* il = static_cast<float*>(D.workspace<1>((size_t)B * img * 4));
-    float* ilT = static_cast<float*>(D.workspace<2>((size_t)B * img * 4));
-    const int prc = proj_plan(g, cv.data(), sv.data(), B, true);
+    float* ilT = rs ? nullptr : static_cast<float*>(D.workspace<2>((size_t)B * img * 4));
     for (int s0 = 0; s0 < nslices; s0 += B) {
         const int nb = std::min(B, nslices - s0);
         const float* src = d_obj + (size_t)s0 * img;
@@ -1026,9 +1034,9 @@ static void radon_device(int dev, float* d_proj, const float* d_obj, const float
         p.y = nullptr; p.wa = nullptr; p.kl_part = nullptr; p.ex_part = nullptr;
         p.cosv = dc.as<double>(); p.sinv = ds.as<double>();
         p.g = g; p.S = nb; p.tlo = 0; p.W = nrays; p.lds_rc = prc;
-        proj_tiles(D, p, cv, sv, prc, nb, budget);
+        proj_tiles(D, p, rs, nb, budget);
         launch_to_interleaved(src, il, nb, Ny, Nx, false, st);
-        if (!p.tile_rs) launch_to_interleaved(src, ilT, nb, Ny, Nx, true, st); // tiles read one orientation
+        if (!rs) launch_to_interleaved(src, ilT, nb, Ny, Nx, true, st);
         if (prc > 0)
             p.lds_rc = tune_pick(proj_tune_key(g, 0, (nb + 3) / 4), proj_rc_cands(g, prc), st, [&](int c) {
                 ProjArgs t = p;
@@ -1110,23 +1118,26 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
     RayGeom rg = ray_geom_em(R, A, n);
 
     const size_t img = (size_t)n * n;
-    // per slice: interleaved image + transpose, staged ratio rows, KL partials
-    const size_t per_slice = img * 8 + (size_t)A * g.width * 4 + (size_t)A * 16;
     int B = blocksize > 0 ? std::min(blocksize, S) : S;
     B = ((B + 3) / 4) * 4;
     const size_t budget = block_budget();
+    int prc = proj_plan(rg, cv.data(), sv.data(), B, true);
+    const int rs = proj_tile_form(rg, cv, sv, prc, budget);
+    // per slice: interleaved image + transpose, staged ratio rows, KL partials
+    const size_t per_slice = img * (rs ? 4 : 8) + (size_t)A * g.width * 4 + (size_t)A * 16;
+    const int whole = B;
     while (B > 4 && (size_t)B * per_slice > budget) B = (((B + 1) / 2 + 3) / 4) * 4;
+    if (prc > 0 && B < whole) prc = proj_plan(rg, cv.data(), sv.data(), B, true);
     const int Gb = B / 4;
 
     float* rows = static_cast<float*>(D.workspace<0>((size_t)Gb * A * g.width * 16));
     float* xil = static_cast<float*>(D.workspace<1>((size_t)Gb * img * 16));
-    float* xT = static_cast<float*>(D.workspace<2>((size_t)Gb * img * 16));
+    float* xT = rs ? nullptr : static_cast<float*>(D.workspace<2>((size_t)Gb * img * 16));
     float* ones = static_cast<float*>(D.workspace<3>(img * 4 + (size_t)A * g.width * 16));
     float* onerows = ones + img;
     // staged-projector ray chunks: the plan's, or the autotuner's choice among
     // powers of two (made on the first block, below); the KL partial slots
     // are sized for the largest candidate
-    int prc = proj_plan(rg, cv.data(), sv.data(), B, true);
     const std::vector<int> rc_cands = prc > 0 ? proj_rc_cands(rg, prc) : std::vector<int>{prc};
     int kslots = proj_kl_slots(A, prc);
     size_t kslots_cap = (size_t)kslots;
@@ -1160,8 +1171,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
 
     ProjArgs tiles; // the tile form's fields
     tiles.g = rg;
-    proj_tiles(D, tiles, cv, sv, prc, B, budget);
-    const bool need_T = !tiles.tile_rs; // tiles read one orientation
+    proj_tiles(D, tiles, rs, B, budget);
 
     // one iteration: projector + ratio (+ KL partials), KL reduction, backprojection + update
     int* counter = reinterpret_cast<int*>(static_cast<char*>(D.workspace<6>(256)));
@@ -1181,7 +1191,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
         if (with_kl) launch_kl_reduce(part, expart, kslots, nb, klo, exo, Kkl, it, graph ? counter : nullptr, s);
         if (kl_only) return;
         BpArgs b;
-        b.q = rows; b.out = xil; b.x = xil; b.norm = ones; b.xt = need_T ? xT : nullptr;
+        b.q = rows; b.out = xil; b.x = xil; b.norm = ones; b.xt = xT;
         b.cA = dcA.as<double>(); b.cB = dcB.as<double>(); b.xc = g.xc; b.c0 = g.c0;
         b.n = n; b.A = A; b.S = nb; b.tlo = g.tlo; b.W = g.width; b.mode = 1; b.chunk = bp_chunk;
         b.q_bytes = (size_t)Gb * A * g.width * 16;
@@ -1240,7 +1250,7 @@ static void eem_device(int dev, float* d_obj, const float* d_tomo, const float* 
         double* klo = Kkl > 0 ? dkl + (size_t)s0 * Kkl : nullptr;
         unsigned long long* exo = Kkl > 0 ? dex + (size_t)s0 * Kkl : nullptr;
         launch_to_interleaved(x, xil, nb, n, n, false, st);
-        if (need_T) launch_to_interleaved(x, xT, nb, n, n, true, st);
+        if (xT) launch_to_interleaved(x, xT, nb, n, n, true, st);
         if (s0 == 0) tune(nb, y);
         for (int it = 0; it < it0; ++it) iteration(it, nb, y, klo, exo, false, st, true);
         if (use_graph) {
@@ -1349,22 +1359,25 @@ static void tem_device(int dev, float* d_obj, const float* d_count, const float*
     RayGeom rg = ray_geom_em(R, A, n);
 
     const size_t img = (size_t)n * n;
-    const size_t per_slice = img * 16 + (size_t)A * g.width * 4;
     int B = blocksize > 0 ? std::min(blocksize, S) : S;
     B = ((B + 3) / 4) * 4;
     const size_t budget = block_budget();
+    int prc = proj_plan(rg, cv.data(), sv.data(), B, true);
+    const int rs = proj_tile_form(rg, cv, sv, prc, budget);
+    const size_t per_slice = img * (rs ? 12 : 16) + (size_t)A * g.width * 4;
+    const int whole = B;
     while (B > 4 && (size_t)B * per_slice > budget) B = (((B + 1) / 2 + 3) / 4) * 4;
+    if (prc > 0 && B < whole) prc = proj_plan(rg, cv.data(), sv.data(), B, true);
     const int Gb = B / 4;
     float* rows = static_cast<float*>(D.workspace<0>((size_t)Gb * A * g.width * 16));
     float* xil = static_cast<float*>(D.workspace<1>((size_t)Gb * img * 16));
-    float* xT = static_cast<float*>(D.workspace<2>((size_t)Gb * img * 16));
+    float* xT = rs ? nullptr : static_cast<float*>(D.workspace<2>((size_t)Gb * img * 16));
     float* normil = static_cast<float*>(D.workspace<3>((size_t)Gb * img * 16));
     float* tmp = static_cast<float*>(D.workspace<5>((size_t)B * img * 4));
-    const int prc = proj_plan(rg, cv.data(), sv.data(), B, true);
 
     ProjArgs tiles;
     tiles.g = rg;
-    proj_tiles(D, tiles, cv, sv, prc, B, budget);
+    proj_tiles(D, tiles, rs, B, budget);
 
     for (int s0 = 0; s0 < S; s0 += B) {
         const int nb = std::min(B, S - s0);
@@ -1381,7 +1394,7 @@ static void tem_device(int dev, float* d_obj, const float* d_count, const float*
         // the rows' margins (bins outside [0, R)) are zero from here on: the
         // projector rewrites only [0, R)
         launch_to_interleaved(x, xil, nb, n, n, false, st);
-        if (!tiles.tile_rs) launch_to_interleaved(x, xT, nb, n, n, true, st);
+        if (xT) launch_to_interleaved(x, xT, nb, n, n, true, st);
         for (int it = 0; it < K; ++it) {
             ProjArgs p;
             p.img = xil; p.imgT = xT; p.out = rows; p.y = d_flat + (size_t)s0 * R; p.wa = dwa.as<float>();
@@ -1394,7 +1407,7 @@ static void tem_device(int dev, float* d_obj, const float* d_count, const float*
                 launch_project(p, 2, st);
             }
             BpArgs b;
-            b.q = rows; b.out = xil; b.x = xil; b.norm = normil; b.norm_il = 1; b.xt = tiles.tile_rs ? nullptr : xT;
+            b.q = rows; b.out = xil; b.x = xil; b.norm = normil; b.norm_il = 1; b.xt = xT;
             b.cA = dcA.as<double>(); b.cB = dcB.as<double>(); b.xc = g.xc; b.c0 = g.c0;
             b.n = n; b.A = A; b.S = nb; b.tlo = g.tlo; b.W = g.width; b.mode = 1;
             b.q_bytes = (size_t)Gb * A * g.width * 16;
@@ -1536,7 +1549,7 @@ static void batch_device(int dev, int nscans, const int* nrays, const int* nangl
             const int G = (S + 3) / 4;
             b->erows.alloc((size_t)G * A * g.width * 16);
             b->xil.alloc((size_t)G * img * 16);
-            b->xT.alloc((size_t)G * img * 16);
+            if (!b->tile_rs) b->xT.alloc((size_t)G * img * 16); // tiles read one orientation
             b->ones.alloc(img * 4 + (size_t)A * g.width * 16);
             b->y.alloc((size_t)S * sino * 4);
             b->x.alloc((size_t)S * img * 4);
@@ -1614,7 +1627,7 @@ static void batch_device(int dev, int nscans, const int* nrays, const int* nangl
             const int G = (S + 3) / 4;
             launch_fill(b->erows.as<float>(), (long long)G * A * g.width * 4, 0.0f, s);
             launch_to_interleaved(b->x.as<float>(), b->xil.as<float>(), S, N, N, false, s);
-            launch_to_interleaved(b->x.as<float>(), b->xT.as<float>(), S, N, N, true, s);
+            if (b->xT.p) launch_to_interleaved(b->x.as<float>(), b->xT.as<float>(), S, N, N, true, s);
         }
     };
     auto enqueue_fbp_scatter = [&](BatchBucket* b, hipStream_t s) {
