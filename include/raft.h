@@ -235,8 +235,9 @@ int raft_fbp_form_info(const float* angles, const float* paramf, const int* para
 /* Host-only planning query of the forward projector (no device work): for
  * the Radon geometry (em = 0: an Ny x Nx image, half extents ax, ay) or the
  * eEM one (em = 1: an Nx x Nx image, Ny = Nx, ax and ay ignored), the number
- * of ray chunks *ray_chunks of the staged (LDS) form, or 0 when the direct
- * form runs (a chunk's staged box would not fit the tile, or RAFT_PROJ_LDS=0).
+ * of ray chunks *ray_chunks of the staged (LDS) form, or 0 when the tile form
+ * runs (a chunk's staged box would not fit: sparse angles) or the direct form
+ * (images below 32 x 32, stretched pixels, or RAFT_PROJ_LDS=0).
  * tile_consts[4] (if non-null) receives the staged form's constants: rays per
  * patch, samples per step, angles per workgroup, staged 16-byte entries.
  * Returns 0 or an error code. */

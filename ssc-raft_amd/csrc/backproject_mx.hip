@@ -17,9 +17,11 @@
 // (8 + 8 + 8 significant bits, truncated, so nothing overflows); products
 // with the selection are exact.  h sums and m + l sums have accumulators of
 // their own.  An h carries 8 bits, so its running sum is exact while it stays
-// below 2^16 times the smallest term, and the m + l sum sits 2^-8 below: the
-// total rounds less than a sum of FP32 values does.  FP16 rows are used as
-// they are, one accumulator, FP32 sums.
+// below 2^16 times the smallest term, and the m + l sum sits 2^-8 below: there the
+// total rounds less than a sum of FP32 values does, and past it the h sum rounds as
+// that would (64 slices of 2048^2: 7.6e-7 from 64 bits, the gather form 9.8e-7).
+// Subnormal pieces count: the instruction does not flush them.  FP16 rows are used
+// as they are, one accumulator, FP32 sums.
 //
 // Workgroup: 8 waves, a tile of 4 x 8 patches (24 x 40 pixels), 4 patches in x
 // per wave (they share the Y part of the coordinate), up to 32 (FP32) or 64
@@ -30,9 +32,10 @@
 // 256, so a read of 4 bins x 32 columns touches every bank once.
 //
 // What bounds it: 64 slices of 2048^2 pixels and 2048 angles move 187 GB from L2
-// into LDS, about 9 TB/s; with that staging switched off the FP32 form takes
-// 15.8 ms of its 21.1.  The rest is the issue of the selection (two waves per
-// SIMD hold the FP32 accumulators: 128 registers each).  The gather kernels take
+// into LDS, about 9 TB/s, and the operand reads keep the LDS pipe at 0.175 wave
+// instructions per clock per CU, as many as it does of 16-byte reads in a loop of
+// nothing else; VALU issue is at 0.36 and the waves wait a third of their cycles
+// (two per SIMD hold the FP32 accumulators: 128 registers each).  The gather kernels take
 // 29.5 ms there (one LDS read per pixel, angle and 4 slices), FP16 rows 23.8 ms
 // against 9.3 here.
 //

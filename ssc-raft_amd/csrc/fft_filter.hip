@@ -13,8 +13,9 @@
 // reads, zeros outside [0, n), into the slice-interleaved layout
 // [group][angle][bin][SB] (SB = 4 for FP32 rows, 8 for FP16 rows).
 //
-// Sizes of 64 M and 512 M bins run k_filter_dif instead: forward passes that
-// leave the spectrum permuted, H in that order, and the same passes back.
+// Twelve sizes, 512, 640, 768, 1024 and 1536, 2048, 2560, 3072, 4096, 5120, 6144, 8192
+// bins, run k_filter_dif instead: forward passes that leave the spectrum permuted, H
+// in that order, and the same passes back.
 //
 // Padded sizes with a prime factor > 5 or n > 16384 run the same circular
 // convolution q[m] = sum_j g[(m - j) mod n] u[j], g = IDFT(H) (built on the host
@@ -195,7 +196,9 @@ __device__ __forceinline__ void fft_pass(float2* z, const Tw& tw, int n, int Ns,
 // (4096, 6144]: two instead of one; 384 threads: four instead of three) and one
 // workgroup's barriers overlap the others' passes (shorter rows: their calls are
 // mostly too small to fill the chip).  16 slices, n = 3072: the polar
-// pass 0.51 -> 0.44 ms, the second inverse transform 0.37 -> 0.31.
+// pass 0.51 -> 0.44 ms, the second inverse transform 0.37 -> 0.31.  The filter that
+// takes one pair a workgroup spills 6 to 8 registers for it at 384 and 512 threads and
+// runs as before (FP16 rows, 8 slices, 200 angles: n = 2400 209 us, 3600 369, 4050 412).
 template <int THREADS> constexpr int fft_wpe() { return THREADS >= 384 && THREADS <= 768 ? 6 : 1; }
 
 struct FftK {
@@ -900,7 +903,8 @@ template <typename OT> void launch_conv(const FilterK& k, const FilterArgs& a, h
     hipLaunchKernelGGL((k_filter_conv<OT>), dim3((unsigned)blocks), dim3(CV_THREADS), lds, st, k, c);
 }
 
-// ---- FP32 rows of n = M0 64 or M0 512 bins (k_filter_dif) -------------------
+// ---- FP32 rows of 64 x 8, 10, 12, 16 and 512 x 3, 4, 5, 6, 8, 10, 12, 16 bins ----
+// ---- (k_filter_dif) ----
 //
 // The same passes in FP32 for the padded row itself (the circular convolution):
 // radix M0 from the sinogram, radix 8 in LDS down to blocks of 8, the product

@@ -2088,7 +2088,9 @@ static void fbp_host(int* gpus, int ngpus, float* obj, float* tomo, float* angle
             if (k >= NB) RAFT_HIP(hipStreamWaitEvent(s_comp.s, ev_d2h[b], 0)); // d_out[b] read by chunk k-NB's copy
             FbpCfg ck = c;
             ck.S = nb;
-            // gather form: a chunk holds few slices, and the copies bound this path
+            // gather form for every chunk, whatever its slices (a chunk of 64 MB holds 16 of
+            // 1024 x 1024 and 64 of 512 x 512, where device calls take the matrix form): an
+            // image does not depend on how a call is cut into chunks
             fbp_run(D, d_out[b], d_in[b], angles, ck, RAFT_STORE_F32, s_comp.s, false, false);
             RAFT_HIP(hipEventRecord(ev_comp[b], s_comp.s));
             RAFT_HIP(hipStreamWaitEvent(s_out.s, ev_comp[b], 0));
@@ -2496,7 +2498,9 @@ int raft_fbp_form_info(const float* angles, const float* paramf, const int* para
         std::vector<float> wa;
         fbp_geometry(c, angles, g, wa);
         if (mx) bp_window_matrix(g);
-        if (form) *form = mx ? 2 : (bp_split_workspace(c.S, c.N, c.A, store) ? 1 : 0);
+        const int SB = (store == RAFT_STORE_F16) ? BP_SLICES_F16 : BP_SLICES_F32;
+        const int B = c.blocksize > 0 ? std::min((c.blocksize + SB - 1) / SB * SB, c.S) : c.S; // slices of a block
+        if (form) *form = mx ? 2 : (bp_split_workspace(B, c.N, c.A, store) ? 1 : 0);
         if (tlo) *tlo = g.tlo;
         if (width) *width = g.width;
     });

@@ -285,7 +285,7 @@ def fbp_form_info(angles, paramf, parami, store="f32"):
 def proj_plan_info(angles, Nx, Ny=None, nrays=None, nslices=4, ax=1.0, ay=1.0, em=False):
     """(ray_chunks, (rays per patch, samples per step, angles per workgroup,
     staged entries)) of the forward projector's plan (host only): ray_chunks
-    > 0 selects the staged (LDS) form, 0 the direct form.  em=True plans the
+    > 0 selects the staged (LDS) form, 0 the tile or direct form.  em=True plans the
     eEM projector of an Nx x Nx image from nrays-bin rows."""
     angles = CNICE(numpy.asarray(angles))
     Ny = Nx if Ny is None else Ny
