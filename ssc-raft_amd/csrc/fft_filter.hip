@@ -569,9 +569,14 @@ __global__ __launch_bounds__(256) void k_filter_direct(FilterK a)
 constexpr int CV_THREADS = 512;
 constexpr int CV_MAX_LEN = 8192; // 147 KB of LDS
 constexpr int CV_MAX_CHUNKS = 16;
-// padded rows from here on: n = 98 takes 10.2 us direct and 13.6 by transforms
-// (320 row pairs), n = 202 43.7 and 22.8 (1440 pairs)
-constexpr int CV_MIN_N = 128;
+// Padded rows from here on, direct -> transforms, us for 19200 row pairs of an FBP:
+// 43 rays padded to 129 160 -> 178, 47 to 141 169 -> 178, 51 to 153 187 -> 181, 67 to
+// 201 452 -> 231; a longer row has more bins to sum, 65 to 130 233 -> 215 (few pairs are
+// 1 to 2 us faster by transforms at all of these).
+constexpr int CV_MIN_N = 136, CV_LEAST_N = 128, CV_LEAST_RAYS = 60;
+// The low-pass keeps N bins of a row, a wave of the direct sum per 64: 57 rays padded to
+// 171 108 -> 178 us, 69 to 138 160 -> 181, 77 to 154 182 -> 179, 67 to 201 230 -> 190.
+constexpr int CV_LEAST_LOWPASS = 300; // waves times padded bins
 // binary orders of magnitude between two rows from which each is summed by itself:
 // below, the larger one's rounding stays 2^8 below an FP32 rounding of the smaller
 constexpr unsigned CV_APART = 20;
@@ -1692,15 +1697,19 @@ bool dif_tables(int n, const std::vector<float2>& H, std::vector<float2>& Hp, st
 ConvPlan conv_plan(int n, int N)
 {
     ConvPlan best;
-    if (n < CV_MIN_N) return best;
+    if (n < CV_LEAST_N || (n < CV_MIN_N && N < CV_LEAST_RAYS)) return best;
     long long cost = 0;
     for (int m : {1, 3, 5})
         for (int len = m * 64, k = 6; len <= CV_MAX_LEN; len *= 2, ++k) {
             const int chunk = std::min(len - N + 1, n);
             if (chunk < 1) continue;
             const int chunks = (n + chunk - 1) / chunk;
-            if (best.len && (long long)chunks * len >= cost) continue;
-            cost = (long long)chunks * len;
+            // of equal cost one long transform instead of two (51 rays padded to 153, 4800
+            // pairs: 85 -> 50 us), but for 8192, of which one workgroup fits a CU (1601 padded
+            // to 4803: 150 us by two of 4096, 228 by one)
+            const long long c = (long long)chunks * len;
+            if (best.len && (c > cost || (c == cost && (chunks >= best.chunks || len > CV_MAX_LEN / 2)))) continue;
+            cost = c;
             best = ConvPlan();
             best.len = len; best.chunk = chunk; best.chunks = chunks;
             if (m > 1) best.radix[best.passes++] = m;
@@ -1711,6 +1720,8 @@ ConvPlan conv_plan(int n, int N)
     if (best.chunks > CV_MAX_CHUNKS) best = ConvPlan();
     return best;
 }
+
+bool conv_pays_lowpass(int n, int N) { return (N + 63) / 64 * n >= CV_LEAST_LOWPASS; }
 
 void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::vector<double>& spec,
                  std::vector<double>& tw, std::vector<double>& edge)

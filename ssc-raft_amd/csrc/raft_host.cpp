@@ -958,6 +958,7 @@ static void lowpass_device(int dev, float* d_tomo, const float* paramf, const in
         fa.wa = dwa.as<float>();
         fa.N = N; fa.A = A; fa.S = nb; fa.npad = c.npad; fa.L = c.L; fa.tlo = c.L; fa.W = N;
         fa.none = 0;
+        if (!conv_pays_lowpass(c.npad, N)) fa.conv = ConvPlan();
         // in place where the filter form writes rows directly (FP32 whole
         // entries with the window in LDS), else through q
         fa.rows = d_tomo + (size_t)s0 * A * N;

@@ -156,6 +156,8 @@ struct ConvPlan {
     int radix[8] = {0};
 };
 ConvPlan conv_plan(int n, int N);
+// whether they are faster than the direct sum where only the N bins of the row are kept
+bool conv_pays_lowpass(int n, int N);
 // its tables from the circular kernel g[n]: spectra [chunks][len] and twiddles
 // [len] (complex), edge sums [2][n]
 void conv_tables(const ConvPlan& p, const double* g, int n, int N, int L, std::vector<double>& spec,
